@@ -1274,19 +1274,27 @@ int64_t dense_extent(const Operand &o, int src, int64_t rows, int64_t k) {
 bool aligned16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 constexpr bool is_nf4_host(int src) { return src == SRC_NF4 || src == SRC_NF4T; }
 
-// Vector (16-byte) operand access needs aligned bases, leading dimensions that are
-// multiples of 8 elements, and 8-multiple extents along each contiguous dimension.
 // Segments the kernels read: both for a two-segment contraction or a grouped launch.
 int operand_segments(const GemmParams &p) { return p.group_tiles > 0 ? 2 : p.nseg; }
 // Columns of segment s's B operand.
 int64_t segment_cols(const GemmParams &p, int s) { return (p.group_tiles > 0 && s == 1) ? p.n1 : p.n; }
+
+// Vector (16-byte) operand access needs aligned bases, leading dimensions that are
+// multiples of 8 elements, and 8-multiple extents along each contiguous dimension.
+// Sources that read 8 (KC) or 32 (NF4) consecutive reduction indices at once.
+constexpr bool along_reduction(int src) { return src == SRC_KC || src == SRC_NF4; }
 
 bool vec_ok(const Problem &pr) {
     const GemmParams &p = pr.p;
     for (int s = 0; s < operand_segments(p); ++s) {
         const Segment &g = p.seg[s];
         const int sa = pr.src[2 * s], sb = pr.src[2 * s + 1];
-        if (g.k % 8) return false;
+        // Only operands whose 16-byte chunks run along the reduction need whole chunks of it:
+        // the output-contiguous ones (KS, KT) and NF4T load one reduction index per chunk and
+        // mask each index past the end, so an odd token count keeps the vector path in the
+        // parameter gradients (MI355X, 4001 tokens, rank 256, 2048 x 8192: the element-wise
+        // loader took 155 us for dA and dB, the vector one 45 us).
+        if (g.k % 8 && (along_reduction(sa) || along_reduction(sb))) return false;
         if (!is_nf4_host(sa) && (!aligned16(g.a.p) || g.a.ld % 8)) return false;
         if (!is_nf4_host(sb) && (!aligned16(g.b.p) || g.b.ld % 8)) return false;
         if ((sa == SRC_KS || sa == SRC_KT) && p.m % 8) return false;

@@ -292,6 +292,34 @@ def test_parameter_gradients_grouped_launch(m, n, k, r):
             assert norm <= 1e-5, (name, norm)
 
 
+@pytest.mark.parametrize("m,n,k,r", [(1, 256, 256, 256), (251, 1024, 768, 256), (4001, 512, 2048, 256),
+                                     (4001, 128, 512, 64), (2055, 136, 72, 8), (515, 264, 264, 128)])
+def test_parameter_gradients_of_a_ragged_token_count(m, n, k, r):
+    """Token counts that are no multiple of 8 take the same kernels as those that are: the
+    result equals, bit for bit, that of the same rows padded with zeros to whole 64-token
+    k-tiles (the plan and the order of the sums depend on the tiles alone; the pairs that
+    straddle a plan's row limit are left out), past rows are not read, and it is within fp32
+    summation error of float64 (1e-5, as above)."""
+    from causal_tuner.kernels.linear import parameter_gradients
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    padded = -(-m // 64) * 64
+    x, dy, low, xa = (torch.randn(padded, width, device="cuda", generator=g).to(torch.bfloat16)
+                      for width in (k, n, r, r))
+    got = torch.full((r, k), float("nan"), device="cuda"), torch.full((n, r), float("nan"), device="cuda")
+    for t in (x, dy, low, xa):
+        t[m:] = float("nan")
+    parameter_gradients(x[:m], dy[:m], *got, low[:m], xa[:m], add=False)
+    for t in (x, dy, low, xa):
+        t[m:] = 0
+    want = torch.empty_like(got[0]), torch.empty_like(got[1])
+    if (m <= 512) == (padded <= 512) and (m <= 2048) == (padded <= 2048):
+        parameter_gradients(x, dy, *want, low, xa, add=False)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    for out, left, right in ((got[0], low, x), (got[1], dy, xa)):
+        _, norm = olora.relative_error(out.cpu(), (left.double().T @ right.double()).cpu())
+        assert norm <= 1e-5
+
+
 @pytest.mark.parametrize("nf4", [False, True])
 def test_merged_weight_is_the_effective_linear_map(nf4):
     """Projection.merged_weight (the merged export, reference checkpointing/io.py:270-280):
