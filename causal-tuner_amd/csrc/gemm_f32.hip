@@ -10,19 +10,25 @@
 // With beta = 0 the destination is never read (garbage or NaN there is ignored).
 //
 // Design: v_mfma_f32_16x16x4_f32 (full fp32 products and sums; no TF32 or reduced-
-// precision step), 128 x 128 output tiles of 4 waves (2 x 2 of 64 x 64), BK = 16, both
-// operands staged k-major in LDS (rows padded by 16 floats so the four k rows a wave
-// reads at once fall in distinct banks), the next k-slice loaded into registers while the
-// current one is multiplied. Every output element is one in-order reduction over k by one
-// lane, so results are deterministic and independent of the grid.
+// precision step), bound by the matrix cores' fp32 rate (157 TFLOP/s at 2.4 GHz; rocBLAS's
+// 8192^3 product reaches 154 on this card). Each operand keeps its stored order in LDS, so no
+// register transposes are needed: [row][32 k] with the bf16 kernels' conflict-free 16-byte
+// swizzle (slot()) when it is contiguous along k, [k][rows] with a column XOR when it is
+// contiguous along its rows. Either way MFMA t of a 16-k slice takes k 4t .. 4t+3 in index
+// order, through conflict-free ds_read_b32 (wider along B's rows). Three tiles by the size of
+// the output (choose()):
+//   128 x 128 and 64 x 64, 4 waves, two stages of 32 k, sums in one chain in index order;
+//   32 x 32, 8 waves that split each 128-k stage between them and add their sums in LDS in a
+//   fixed order: an adapter's products (1000 x 64 over 2048) give few tiles, and the split
+//   reduction inside the workgroup keeps the chip busy without a workspace.
+// Every output element is a fixed-order reduction, so results repeat bit for bit.
 
-#include "common.hpp"
+#include <type_traits>
+
+#include "gemm_common.hpp"
 
 namespace ct {
 namespace {
-
-constexpr int kBM = 128, kBN = 128, kBK = 16, kPad = 16, kThreadsF32 = 256;
-constexpr int kRow = kBM + kPad;  // floats per k row of a staged tile (kBM == kBN)
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -32,137 +38,264 @@ struct F32Args {
     const float *a, *b, *bias;
     float *c;
     int64_t lda, ldb, ldc, m, n, k;
-    int trans_a, trans_b, beta, vec_a, vec_b;
+    int tiles_m, tiles_n, beta, vec_c;
 };
 
-// One operand's k-slice [k0, k0 + 16) of the tile rows [r0, r0 + 128) into registers:
-// eight values per thread. `rows_fast` says the stored matrix is contiguous along the tile
-// rows (m of A when trans_a, n of B when !trans_b); otherwise it is contiguous along k.
-struct Slice {
-    float v[8];
-};
+// One operand's tile of a stage of KD * 32 reduction indices, ROWS rows, moved in 16-byte
+// chunks that keep the stored order: KFAST, stored [rows, k], goes to [KD][ROWS][32 k] with
+// tile row n at LDS row frag_row<FRAG>(n); otherwise stored [k, rows], it goes to
+// [k][ROWS], columns XORed with shift(k). VEC: 16-byte loads (aligned base, pitch and
+// contiguous extent in multiples of 4).
+template <int ROWS, int KD, int THREADS, bool KFAST, bool VEC, int FRAG>
+struct Tile {
+    static constexpr int kPer = ROWS * 8 * KD / THREADS;
+    static_assert(kPer >= 1 && kPer * THREADS == ROWS * 8 * KD, "whole chunks per thread");
+    f32x4 v[kPer];
 
-__device__ __forceinline__ void load_slice(const float *p, int64_t ld, bool rows_fast, bool vec, int64_t r0,
-                                           int64_t rows, int64_t k0, int64_t kdim, int tid, Slice &s) {
-    if (rows_fast) {
-        // stored [k, rows]: thread t covers k row (t / 32) * 2 + h, rows 4 (t % 32) .. +3
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int kk = (tid / 32) * 2 + h, rr = (tid % 32) * 4;
-            const int64_t kg = k0 + kk, rg = r0 + rr;
-            if (vec && kg < kdim && rg + 3 < rows) {
-                const f32x4 q = *reinterpret_cast<const f32x4 *>(p + kg * ld + rg);
-                s.v[4 * h + 0] = q[0], s.v[4 * h + 1] = q[1], s.v[4 * h + 2] = q[2], s.v[4 * h + 3] = q[3];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s.v[4 * h + j] = (kg < kdim && rg + j < rows) ? p[kg * ld + rg + j] : 0.f;
-            }
+    // Rows 4t .. 4t+3 of a [k][ROWS] tile start on distinct 16-bank groups under this XOR
+    // (a row of 32 floats spans half the banks, so every second row moves).
+    __device__ __forceinline__ static int shift(int k) { return ROWS >= 64 ? (k & 3) << 4 : (k & 2) << 3; }
+
+    __device__ __forceinline__ static void place(int tid, int i, int &row, int &kk) {
+        const int id = tid + i * THREADS;
+        if constexpr (KFAST) {
+            row = id / (8 * KD);
+            kk = (id % (8 * KD)) * 4;
+        } else {
+            row = (id % (ROWS / 4)) * 4;
+            kk = id / (ROWS / 4);
         }
-    } else {
-        // stored [rows, k]: thread t covers row (t / 4) + 64 h, k 4 (t % 4) .. +3
+    }
+    __device__ __forceinline__ void load(const float *p, int64_t ld, int64_t r0, int64_t rows, int64_t k0,
+                                         int64_t kdim, int tid) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int rr = tid / 4 + 64 * h, kk = (tid % 4) * 4;
-            const int64_t kg = k0 + kk, rg = r0 + rr;
-            if (vec && rg < rows && kg + 3 < kdim) {
-                const f32x4 q = *reinterpret_cast<const f32x4 *>(p + rg * ld + kg);
-                s.v[4 * h + 0] = q[0], s.v[4 * h + 1] = q[1], s.v[4 * h + 2] = q[2], s.v[4 * h + 3] = q[3];
+        for (int i = 0; i < kPer; ++i) {
+            int row, kk;
+            place(tid, i, row, kk);
+            const int64_t rg = r0 + row, kg = k0 + kk;
+            const int64_t left = KFAST ? (rg < rows ? kdim - kg : 0) : (kg < kdim ? rows - rg : 0);
+            const float *src = KFAST ? p + rg * ld + kg : p + kg * ld + rg;
+            if constexpr (VEC) {
+                v[i] = left > 0 ? *reinterpret_cast<const f32x4 *>(src) : f32x4{0.f, 0.f, 0.f, 0.f};
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) s.v[4 * h + j] = (rg < rows && kg + j < kdim) ? p[rg * ld + kg + j] : 0.f;
+                for (int j = 0; j < 4; ++j) v[i][j] = j < left ? src[j] : 0.f;
             }
         }
     }
-}
+    __device__ __forceinline__ void store(f32x4 *stage, int tid) const {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            int row, kk;
+            place(tid, i, row, kk);
+            if constexpr (KFAST) stage[(kk >> 5) * ROWS * 8 + slot(frag_row<FRAG>(row), (kk & 31) >> 2)] = v[i];
+            else stage[(kk * ROWS + (row ^ shift(kk))) / 4] = v[i];
+        }
+    }
+    // Fragment f (of FRAGS) of the 16 * FRAGS rows from w0, for MFMA t of slice `slice` (k 16
+    // slice + 4t + lane / 16): rows w0 + 16 f + lane % 16 with FRAG = 1, else rows
+    // w0 + FRAG (lane % 16) + f.
+    template <int FRAGS>
+    __device__ __forceinline__ static void fragments(const f32x4 *stage, int w0, int slice, int t, int lane,
+                                                     float (&out)[FRAGS]) {
+        const float *base = reinterpret_cast<const float *>(stage);
+        const int g = lane >> 4, c = lane & 15;
+        if constexpr (KFAST) {
+#pragma unroll
+            for (int f = 0; f < FRAGS; ++f)
+                out[f] = base[((slice >> 1) * ROWS * 8 + slot(w0 + f * 16 + c, (slice & 1) * 4 + t)) * 4 + g];
+        } else if constexpr (FRAG == 1) {
+#pragma unroll
+            for (int f = 0; f < FRAGS; ++f)
+                out[f] = base[(16 * slice + 4 * t + g) * ROWS + ((w0 + f * 16 + c) ^ shift(g))];
+        } else {
+            typedef float vec __attribute__((ext_vector_type(FRAG)));
+            const vec q = *reinterpret_cast<const vec *>(base + (16 * slice + 4 * t + g) * ROWS +
+                                                         ((w0 + FRAG * c) ^ shift(g)));
+#pragma unroll
+            for (int f = 0; f < FRAGS; ++f) out[f] = q[f];
+        }
+    }
+};
 
-// Registers -> the k-major LDS tile t[k][row].
-__device__ __forceinline__ void store_slice(float *t, bool rows_fast, int tid, const Slice &s) {
-    if (rows_fast) {
+// Output columns col .. col + N - 1 of one row: + bias, + C when beta.
+template <int N>
+__device__ __forceinline__ void write_row(const F32Args &g, int64_t row, int64_t col, const float (&acc)[N]) {
+    if (row >= g.m || col >= g.n) return;
+    float *c = g.c + row * g.ldc + col;
+    if (N > 1 && g.vec_c && col + N <= g.n) {
+        typedef float vec __attribute__((ext_vector_type(N > 1 ? N : 2)));
+        vec w;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int kk = (tid / 32) * 2 + h, rr = (tid % 32) * 4;
-            *reinterpret_cast<f32x4 *>(t + kk * kRow + rr) =
-                f32x4{s.v[4 * h], s.v[4 * h + 1], s.v[4 * h + 2], s.v[4 * h + 3]};
-        }
-    } else {
+        for (int j = 0; j < N; ++j) w[j] = acc[j] + (g.bias ? g.bias[col + j] : 0.f);
+        if (g.beta) w = *reinterpret_cast<const vec *>(c) + w;
+        *reinterpret_cast<vec *>(c) = w;
+        return;
+    }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int rr = tid / 4 + 64 * h, kk = (tid % 4) * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) t[(kk + j) * kRow + rr] = s.v[4 * h + j];
-        }
+    for (int j = 0; j < N; ++j) {
+        if (col + j >= g.n) break;
+        const float v = acc[j] + (g.bias ? g.bias[col + j] : 0.f);
+        c[j] = g.beta ? c[j] + v : v;
     }
 }
 
-__global__ __launch_bounds__(kThreadsF32) void gemm_f32(const F32Args g) {
-    __shared__ float sa[2][kBK * kRow];
-    __shared__ float sb[2][kBK * kRow];
+// BM x BN tile; WAVES_M x WAVES_N waves over it, KW of them along the reduction: a stage
+// holds KD * 32 reduction indices in 2 KD slices of 16, of which wave group w multiplies
+// slices w * 2 KD / KW and on.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int KW, int KD, bool AK, bool BKF, bool VEC>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KW) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f32(
+    const F32Args g) {
+    constexpr int THREADS = 64 * WAVES_M * WAVES_N * KW;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
+    constexpr int kSlices = 2 * KD / KW, kDepth = 32 * KD;
+    constexpr int kStage = (BM + BN) * 8 * KD;  // 16-byte units
+    static_assert(kSlices >= 1, "every wave group has a slice");
+    static_assert(KW == 1 || (WAVES_M == 1 && WAVES_N == 1 && KW * BM * BN * 4 <= 2 * kStage * 16 &&
+                              BM * BN % THREADS == 0),
+                  "the groups' sums fit the stages");
+    __shared__ f32x4 lds[2 * kStage];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t tiles_n = (g.n + kBN - 1) / kBN;
-    const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * kBM, n0 = (int64_t)(blockIdx.x % tiles_n) * kBN;
-    const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-    const bool a_rows_fast = g.trans_a != 0, b_rows_fast = g.trans_b == 0;
+    const int group = KW > 1 ? wave : 0;
+    const int wm = KW > 1 ? 0 : (wave % WAVES_M) * WM, wn = KW > 1 ? 0 : (wave / WAVES_M) * WN;
 
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Tile order: contiguous ranges per XCD, in groups of 8 row tiles that share B panels.
+    constexpr int kXcds = 8, kGroupM = 8;
+    const int tiles = g.tiles_m * g.tiles_n, xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
+    const int per = (tiles + kXcds - 1) / kXcds, tall = tiles % kXcds == 0 ? kXcds : tiles % kXcds;
+    const int rid = xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int gm = g.tiles_m < kGroupM ? g.tiles_m : kGroupM;
+    const int span = gm * g.tiles_n, first_m = rid / span * gm;
+    const int gsize = g.tiles_m - first_m < gm ? g.tiles_m - first_m : gm;
+    const int64_t m0 = (int64_t)(first_m + rid % span % gsize) * BM, n0 = (int64_t)(rid % span / gsize) * BN;
 
-    const int64_t steps = (g.k + kBK - 1) / kBK;
-    Slice la, lb;
-    if (steps > 0) {
-        load_slice(g.a, g.lda, a_rows_fast, g.vec_a, m0, g.m, 0, g.k, tid, la);
-        load_slice(g.b, g.ldb, b_rows_fast, g.vec_b, n0, g.n, 0, g.k, tid, lb);
-        store_slice(sa[0], a_rows_fast, tid, la);
-        store_slice(sb[0], b_rows_fast, tid, lb);
-    }
-    __syncthreads();
-    for (int64_t s = 0; s < steps; ++s) {
-        const int cur = (int)(s & 1);
-        const bool more = s + 1 < steps;
-        if (more) {
-            load_slice(g.a, g.lda, a_rows_fast, g.vec_a, m0, g.m, (s + 1) * kBK, g.k, tid, la);
-            load_slice(g.b, g.ldb, b_rows_fast, g.vec_b, n0, g.n, (s + 1) * kBK, g.k, tid, lb);
-        }
-        const float *ta = sa[cur], *tb = sb[cur];
+    f32x4 acc[FM][FN];
 #pragma unroll
-        for (int kk = 0; kk < kBK; kk += 4) {
-            const int kr = kk + lane / 16;
-            float af[4], bf[4];
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = ta[kr * kRow + wm + i * 16 + (lane & 15)];
+        for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // SETS register sets per operand: step s stores tile s + 1 to the other stage before its
+    // products and loads tile s + 1 + SETS into the set that freed, so a load has SETS steps
+    // to arrive. Two where registers allow it: the 128 x 128 tile would spill.
+    constexpr int SETS = BM >= 128 ? 1 : 2;
+    using TileA = Tile<BM, KD, THREADS, AK, VEC, 1>;
+    using TileB = Tile<BN, KD, THREADS, BKF, VEC, FN>;
+    TileA la[SETS];
+    TileB lb[SETS];
+    const int64_t steps = (g.k + kDepth - 1) / kDepth;
+    const auto load = [&](auto set, int64_t s) {
+        la[set].load(g.a, g.lda, m0, g.m, s * kDepth, g.k, tid);
+        lb[set].load(g.b, g.ldb, n0, g.n, s * kDepth, g.k, tid);
+    };
+    const auto store = [&](auto set, int stage) {
+        la[set].store(lds + stage * kStage, tid);
+        lb[set].store(lds + stage * kStage + BM * 8 * KD, tid);
+    };
+    const auto step = [&](auto cur, int64_t s) {
+        constexpr int nxt = decltype(cur)::value ^ 1;
+        const std::integral_constant<int, nxt % SETS> set{};
+        if (s + 1 < steps) store(set, nxt);
+        if (s + 1 + SETS < steps) load(set, s + 1 + SETS);
+        const f32x4 *sa = lds + decltype(cur)::value * kStage, *sb = sa + BM * 8 * KD;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) bf[j] = tb[kr * kRow + wn + j * 16 + (lane & 15)];
+        for (int q = 0; q < kSlices; ++q) {
+            const int slice = group * kSlices + q;
+            float af[4][FM], bf[4][FN];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int t = 0; t < 4; ++t) {
+                TileA::template fragments<FM>(sa, wm, slice, t, lane, af[t]);
+                TileB::template fragments<FN>(sb, wn, slice, t, lane, bf[t]);
+            }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma_f32(af[i], bf[j], acc[i][j]);
-        }
-        if (more) {
-            store_slice(sa[cur ^ 1], a_rows_fast, tid, la);
-            store_slice(sb[cur ^ 1], b_rows_fast, tid, lb);
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] = mfma_f32(af[t][i], bf[t][j], acc[i][j]);
         }
         __syncthreads();
+    };
+    const std::integral_constant<int, 0> even{};
+    const std::integral_constant<int, 1> odd{};
+    if (steps > 0) {
+        load(even, 0);
+        if (SETS > 1 && steps > 1) load(std::integral_constant<int, SETS - 1>{}, 1);
+        store(even, 0);
+        if (steps > SETS) load(even, SETS);
+        __syncthreads();
+        int64_t s = 0;
+        for (; s + 1 < steps; s += 2) {
+            step(even, s);
+            step(odd, s + 1);
+        }
+        if (s < steps) step(even, s);
     }
 
-    // lane l holds rows 4 (l / 16) + e of each 16-row block and column l % 16
+    // Lane l holds rows 4 (l / 16) + e of each 16-row block and, of the wave's columns,
+    // FN (l % 16) + j.
+    if constexpr (KW > 1) {
+        float *sums = reinterpret_cast<float *>(lds);  // free: every wave has left the loop
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int64_t col = n0 + wn + j * 16 + (lane & 15);
-        if (col >= g.n) continue;
-        const float bias = g.bias ? g.bias[col] : 0.f;
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    sums[group * BM * BN + (i * 16 + (lane >> 4) * 4 + e) * BN + (lane & 15) * FN + j] = acc[i][j][e];
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < BM * BN / THREADS; ++o) {
+            const int at = o * THREADS + tid;
+            float v[1] = {sums[at]};
+#pragma unroll
+            for (int w = 1; w < KW; ++w) v[0] += sums[w * BM * BN + at];
+            write_row<1>(g, m0 + at / BN, n0 + at % BN, v);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int64_t row = m0 + wm + i * 16 + (lane >> 4) * 4 + e;
-                if (row >= g.m) continue;
-                float *c = g.c + row * g.ldc + col;
-                const float v = acc[i][j][e] + bias;
-                *c = g.beta ? *c + v : v;
+                float v[FN];
+#pragma unroll
+                for (int j = 0; j < FN; ++j) v[j] = acc[i][j][e];
+                write_row<FN>(g, m0 + wm + i * 16 + (lane >> 4) * 4 + e, n0 + wn + (lane & 15) * FN, v);
             }
     }
+}
+
+enum Shape { LARGE, MEDIUM, SMALL };
+constexpr int kEdge[3] = {128, 64, 32};
+
+// 128 x 128 tiles once they give every CU a workgroup, 64 x 64 ones likewise, and the split
+// 32 x 32 tile for everything smaller, unless the reduction fits one of its stages (nothing to
+// split: 64 x 64 tiles, which also keep such sums in one chain). MI355X, one launch
+// (trans_b = 1): 4096 x 4096 x 4096 1077 us, 1198 on 64 x 64 tiles (1243 with the previous
+// 128 x 128 kernel of b32-staged 16-k slices); 1000 x 2048 x 2048 98, 109 on 32 x 32 (219);
+// 1000 x 64 x 2048 17 us, 57 on 64 x 64 (215); 64 x 2048 x 1000 10 us, 29 (109).
+Shape choose(int64_t m, int64_t n, int64_t k) {
+    if (cdiv(m, 128) * cdiv(n, 128) >= 256) return LARGE;
+    return cdiv(m, 64) * cdiv(n, 64) >= 256 || k <= 128 ? MEDIUM : SMALL;
+}
+
+template <bool AK, bool BKF, bool VEC>
+void launch_shape(Shape shape, const F32Args &g, hipStream_t s) {
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
+    if (shape == LARGE) gemm_f32<128, 128, 2, 2, 1, 1, AK, BKF, VEC><<<grid, dim3(256), 0, s>>>(g);
+    else if (shape == MEDIUM) gemm_f32<64, 64, 2, 2, 1, 1, AK, BKF, VEC><<<grid, dim3(256), 0, s>>>(g);
+    else gemm_f32<32, 32, 1, 1, 8, 4, AK, BKF, VEC><<<grid, dim3(512), 0, s>>>(g);
+}
+
+template <bool AK, bool BKF>
+void launch_vec(Shape shape, bool vec, const F32Args &g, hipStream_t s) {
+    if (vec) launch_shape<AK, BKF, true>(shape, g, s);
+    else launch_shape<AK, BKF, false>(shape, g, s);
+}
+
+// 16-byte loads: aligned base, pitch and extent of the contiguous dimension in multiples of 4.
+bool operand_vec(const float *p, int64_t ld, int64_t contiguous) {
+    return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && contiguous % 4 == 0;
 }
 
 }  // namespace
@@ -175,18 +308,23 @@ extern "C" int ct_gemm_f32(const float *a, int64_t lda, int32_t trans_a, const f
     if (m < 0 || n < 0 || k < 0) return -CT_EINVAL_SHAPE;
     if (m == 0 || n == 0) return 0;
     if (!c || (k > 0 && (!a || !b))) return -CT_EINVAL_POINTER;
-    const int64_t arows = trans_a ? k : m, acols = trans_a ? m : k;
-    const int64_t brows = trans_b ? n : k, bcols = trans_b ? k : n;
-    if (ldc < n || (k > 0 && (lda < acols || ldb < bcols)) || arows < 0 || brows < 0) return -CT_EINVAL_SHAPE;
+    const int64_t acols = trans_a ? m : k, bcols = trans_b ? k : n;
+    if (ldc < n || (k > 0 && (lda < acols || ldb < bcols))) return -CT_EINVAL_SHAPE;
     F32Args g{};
     g.a = a, g.b = b, g.bias = bias, g.c = c;
     g.lda = lda, g.ldb = ldb, g.ldc = ldc, g.m = m, g.n = n, g.k = k;
-    g.trans_a = trans_a != 0, g.trans_b = trans_b != 0, g.beta = beta != 0;
-    g.vec_a = reinterpret_cast<uintptr_t>(a) % 16 == 0 && lda % 4 == 0;
-    g.vec_b = reinterpret_cast<uintptr_t>(b) % 16 == 0 && ldb % 4 == 0;
-    const int64_t tiles = ((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
-    if (tiles > 0x7fffffff) return -CT_EINVAL_SHAPE;
-    gemm_f32<<<dim3((unsigned)tiles), dim3(kThreadsF32), 0, stream>>>(g);
+    g.beta = beta != 0;
+    g.vec_c = reinterpret_cast<uintptr_t>(c) % 16 == 0 && ldc % 4 == 0;
+    const Shape shape = choose(m, n, k);
+    const int64_t tm = cdiv(m, kEdge[shape]), tn = cdiv(n, kEdge[shape]);
+    if (tm * tn > 0x7fffffff) return -CT_EINVAL_SHAPE;
+    g.tiles_m = (int)tm;
+    g.tiles_n = (int)tn;
+    const bool vec = operand_vec(a, lda, acols) && operand_vec(b, ldb, bcols);
+    if (trans_a && trans_b) launch_vec<false, true>(shape, vec, g, stream);
+    else if (trans_a) launch_vec<false, false>(shape, vec, g, stream);
+    else if (trans_b) launch_vec<true, true>(shape, vec, g, stream);
+    else launch_vec<true, false>(shape, vec, g, stream);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;  // a positive HIP error code
 }

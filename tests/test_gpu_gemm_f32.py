@@ -47,6 +47,27 @@ def test_layouts_against_float64(m, n, k, trans_l, trans_r):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("m,n,k", [(1000, 64, 2048), (31, 33, 129), (65, 4, 4095), (1028, 1020, 132), (2049, 2044, 36),
+                                   (33, 1000, 128)])
+@pytest.mark.parametrize("trans_l", [False, True])
+@pytest.mark.parametrize("trans_r", [False, True])
+def test_every_tile_with_bias_and_accumulation(m, n, k, trans_l, trans_r):
+    """The three output tiles (32 x 32 with the reduction split inside the workgroup, 64 x 64,
+    128 x 128) at partial tiles and stages, bias and accumulation in one call sequence, against
+    float64."""
+    from causal_tuner.kernels.linear import mm_f32
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    left = torch.randn(k, m, device="cuda", generator=g).T if trans_l else torch.randn(m, k, device="cuda", generator=g)
+    right = torch.randn(n, k, device="cuda", generator=g).T if trans_r else torch.randn(k, n, device="cuda", generator=g)
+    bias = torch.randn(n, device="cuda", generator=g)
+    out = torch.full((m, n), float("nan"), device="cuda")
+    mm_f32(left, right, out, bias=bias)
+    want = _ref(left, right, bias=bias)
+    _close(out, want, k)
+    mm_f32(left, right, out, add=True)
+    _close(out, want + _ref(left, right), k)
+
+
 def test_bias_accumulate_and_strided_views():
     from causal_tuner.kernels.linear import mm_f32
     g = torch.Generator(device="cuda").manual_seed(3)
