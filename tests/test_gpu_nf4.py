@@ -200,3 +200,38 @@ def test_device_quantizer_round_trip_large():
     gap = float((torch.tensor(onf4.NF4_CODE[1:]) - torch.tensor(onf4.NF4_CODE[:-1])).max())
     # the decoded scale differs from absmax by the 8-bit second level: allow 2% of it
     assert bool((err <= scale * (gap / 2 + 0.02)).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("count,blocksize", [(8, 8), (64, 64), (8 * 257, 16), (2048 * 3 + 72, 64), (20480, 256), (20488, 512),
+                                             (20488, 1024)])
+def test_contiguous_quantizer_codes_every_value_as_the_oracle(count, blocksize, dtype):
+    """The first level's contiguous kernel (blocks of 8 to 512 elements, counts in multiples of
+    8) at partial blocks, waves and workgroups, beside 1024-element blocks (a lane per block):
+    byte for byte against the oracle on values at, just below and just above every decision
+    midpoint, zero blocks, infinities and NaN."""
+    from causal_tuner.quant.nf4 import nf4_thresholds, quantize_nf4
+    g = torch.Generator().manual_seed(count + blocksize)
+    values = torch.rand(count, generator=g) * 2 - 1
+    mids = nf4_thresholds()
+    edges = torch.cat((mids, torch.nextafter(mids, mids - 1), torch.nextafter(mids, mids + 1)))
+    values[1:1 + min(len(edges), count - 1)] = edges[:count - 1]
+    values[::blocksize] = 1.0   # the block maximum, so that values divide to themselves
+    if count > 4 * blocksize:
+        values[blocksize:2 * blocksize] = 0
+        values[2 * blocksize + 1], values[3 * blocksize + 2] = float("inf"), float("nan")
+    values = values.to(dtype)
+    packed, state = quantize_nf4(values.cuda(), blocksize=blocksize, compress_statistics=False)
+    with np.errstate(all="ignore"):
+        want_packed, want = _oracle_quantize(values, blocksize, False)
+    # the oracle's maximum over a block with a NaN is NaN, the kernels' ignores it: such blocks
+    # are compared apart
+    clean = np.ones(-(-count // blocksize), dtype=bool)
+    clean[torch.isnan(values).nonzero().flatten().numpy() // blocksize] = False
+    keep = clean.repeat(blocksize // 2)[:count // 2]
+    np.testing.assert_array_equal(packed.cpu().numpy().reshape(-1)[keep], want_packed[keep])
+    np.testing.assert_array_equal(state.absmax.cpu().numpy()[clean], want["absmax"][clean])
+    if count > 4 * blocksize:   # NaN takes the last code
+        at = 3 * blocksize + 2
+        byte = int(packed.cpu().view(-1)[at // 2])
+        assert (byte >> 4 if at % 2 == 0 else byte & 15) == 15
