@@ -54,6 +54,25 @@ def test_trig_tables_in_float32_with_bf16_activations():
     assert torch.equal(y.cpu().float(), _oracle(x, c, s, 16, torch.bfloat16))
 
 
+@pytest.mark.parametrize("trig", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens,heads,head_dim,half,pitch", [
+    (1, 1, 8, 4, 8), (257, 5, 24, 8, 120), (33, 2, 64, 12, 136), (33, 2, 64, 6, 128), (7, 3, 16, 8, 52),
+    (9, 1, 128, 4, 128)])
+def test_inverse_rotation_of_pitched_tiles(tokens, heads, head_dim, half, pitch, trig):
+    """inverse_rope_tile between matrices of any pitch, bit for bit: runs of 8 channels (all
+    rotating or all passing) and, at 6 rotated pairs or a pitch of 52, the pair kernel."""
+    from causal_tuner.kernels.core_cuda import inverse_rope_tile
+    g = torch.Generator().manual_seed(tokens + half)
+    width = heads * head_dim
+    x = torch.randn(tokens, pitch, generator=g).to(torch.bfloat16)
+    c, s = _tables(tokens, half, trig, seed=5)
+    out = torch.full((tokens, pitch + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    got = inverse_rope_tile(x.cuda()[:, :width], c.cuda(), s.cuda(), head_dim, out[:, :width])
+    want = _oracle(x[:, :width].reshape(tokens, heads, head_dim), c, s, head_dim, torch.bfloat16, inverse=True)
+    assert torch.equal(got.cpu().float().reshape(want.shape), want)
+    assert bool((out[:, width:] == 7).all())
+
+
 def test_rotate_owned_qk_in_place_touches_only_rotated_channels():
     from causal_tuner.kernels.core_cuda import rotate_owned_qk
     rows, head_dim, half = 4099, 128, 32
