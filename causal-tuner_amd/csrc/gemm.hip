@@ -313,7 +313,9 @@ struct SegmentRunner {
 // buffer loads: the hardware range check returns zeros past num_records, and an invalid
 // lane is pointed past the range, so the k-loop body has no branches and the compiler can
 // interleave loads, LDS traffic, NF4 decoding and MFMA within one basic block.
-template <int SRC, int ROWS, int FRAG, int THREADS>
+// LEAN (KC only) keeps one register for the reduction column that all of a lane's loads share,
+// for runners short of registers; the other form leaves the tuned kernels' allocation alone.
+template <int SRC, int ROWS, int FRAG, int THREADS, bool LEAN = false>
 struct Fast;
 
 // KC: each wave instruction moves 64 x 16 bytes = 8 tile rows x 8 chunks; lane l owns slot
@@ -322,15 +324,15 @@ struct Fast;
 // MI355X at M=8192 this beat loading straight into LDS (buffer_load ... lds) by 5-20%, as
 // the LDS form needs an M0 write per wave instruction and must complete before the barrier
 // that publishes the stage, while register staging lets the loads run across it.
-template <int ROWS, int FRAG, int THREADS>
-struct Fast<SRC_KC, ROWS, FRAG, THREADS> {
+template <int ROWS, int FRAG, int THREADS, bool LEAN>
+struct Fast<SRC_KC, ROWS, FRAG, THREADS, LEAN> {
     static constexpr int kWaves = THREADS / 64;
     static constexpr int kInstr = ROWS / (8 * kWaves);
     static constexpr int kVmem = kInstr, kWrites = kInstr;  // per tile, per lane
     static_assert(kInstr >= 1, "tile too small for the workgroup");
     __amdgpu_buffer_rsrc_t r;
     uint32_t off[kInstr];  // byte offset of the lane's chunk at k0 = 0
-    int kc[kInstr];        // the lane's first reduction column within the tile
+    int kc[LEAN ? 1 : kInstr];  // the lane's first reduction column within the tile
     int kext;              // reduction extent (< 2^31: fast_ok bounds every operand)
     int wave;
     __device__ __forceinline__ void init(const Operand &o, int64_t rows, int64_t kext_, int64_t r0, int tid) {
@@ -345,7 +347,7 @@ struct Fast<SRC_KC, ROWS, FRAG, THREADS> {
             int srow, c;
             slot_coords((wave * kInstr + i) * 64 + lane, srow, c);
             const int row = frag_row_inv<FRAG>(srow);
-            kc[i] = c * 8;
+            kc[LEAN ? 0 : i] = c * 8;
             off[i] = (uint32_t)((row * o.ld + c * 8) * 2);
         }
     }
@@ -353,7 +355,7 @@ struct Fast<SRC_KC, ROWS, FRAG, THREADS> {
     __device__ __forceinline__ void issue(uint4 *, int64_t k0) {
 #pragma unroll
         for (int i = 0; i < kInstr; ++i) {
-            const uint32_t o = ((int)k0 + kc[i] < kext) ? off[i] + (uint32_t)(k0 * 2) : kOOB;
+            const uint32_t o = ((int)k0 + kc[LEAN ? 0 : i] < kext) ? off[i] + (uint32_t)(k0 * 2) : kOOB;
             v[i] = buf_load16(r, o);
         }
     }
@@ -503,6 +505,30 @@ struct Fast<SRC_NF4, ROWS, FRAG, THREADS> {
             a2[i] = __builtin_bit_cast(float, buf_load4(r2, ok[i] ? (g >> lb2) * 4 : kOOB));
         }
     }
+    // The decode in four pieces of 8 elements, for runners that spread it over a k-step: the
+    // code-book reads of piece P, then (when they have arrived) its products and LDS store.
+    static constexpr int kPieces = 4;
+    float scale;
+    __device__ __forceinline__ void decode_scales(const float *lcode2, float offset) {
+        static_assert(kPer == 1, "one unit per lane");
+        const float decoded = lcode2[qa[0] & 255u] * a2[0] + offset;  // read unconditionally: no branch
+        scale = ok[0] ? decoded : 0.f;
+    }
+    template <int P>
+    __device__ __forceinline__ void lookup(const float *lcode, float (&v)[8]) const {
+        const uint32_t d = P == 0 ? q[0].x : P == 1 ? q[0].y : P == 2 ? q[0].z : q[0].w;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            v[2 * b] = lcode[(d >> (8 * b + 4)) & 15u];
+            v[2 * b + 1] = lcode[(d >> (8 * b)) & 15u];
+        }
+    }
+    template <int P>
+    __device__ __forceinline__ void finish(uint4 *stage, const float (&v)[8]) const {
+        stage[slot(frag_row<FRAG>(row[0]), half[0] * 4 + P)] =
+            make_uint4(pack_bf16x2(v[0] * scale, v[1] * scale), pack_bf16x2(v[2] * scale, v[3] * scale),
+                       pack_bf16x2(v[4] * scale, v[5] * scale), pack_bf16x2(v[6] * scale, v[7] * scale));
+    }
     __device__ __forceinline__ void commit(uint4 *stage, const float *lcode, const float *lcode2,
                                            float offset) const {
 #pragma unroll
@@ -629,7 +655,10 @@ struct FastRunner {
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
     static constexpr int FM = WM / 16, FN = WN / 16;
     static constexpr int KS = kBK / 32;
-    using LA = Fast<SA, BM, 1, THREADS>;
+    // 256 x 256 tiles of 8 waves: the NF4 loader's unit fits packed_step's pieces. (The same
+    // step over NF4T spilled registers: 208 -> 259 us for the dx product of 251 x 24576.)
+    static constexpr bool kPacked = SA == SRC_KC && SB == SRC_NF4 && BN == 256 && THREADS == 512;
+    using LA = Fast<SA, BM, 1, THREADS, kPacked>;
     using LB = Fast<SB, BN, FN, THREADS>;
 
     // One k-step: MFMAs over stage `cur` while the registers' tile goes into stage `nxt`
@@ -670,6 +699,56 @@ struct FastRunner {
         __syncthreads();
     }
 
+    // The k-step over a packed B: the decode of the next tile's 32 elements per lane is spread
+    // over the columns, each piece's code-book reads two columns ahead of its products, and
+    // every column's order is fixed, so that lookups, conversions and stores run between the
+    // MFMAs. Left to the scheduler (step above, whose group pattern does not know the lookups)
+    // the phases ran one after the other: MFMA 29%, VALU 28% and LDS 40% busy, none of them
+    // bound (251 rows, 24576 -> 6144: 116 us, 106 here; 128 rows 94, 82). Same values and sums.
+    template <int J>
+    __device__ __forceinline__ static void packed_column(LA &la, const LB &now, const uint4 *cur, uint4 *nxt,
+                                                         const uint4 (&af)[KS][FM], uint4 (&bf)[2][KS],
+                                                         float (&v)[8], f32x4 (&acc)[FM][FN], const float *lcode,
+                                                         int lane, int wn0) {
+        if constexpr (J < FN) {
+            if constexpr (J + 1 < FN) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    bf[(J + 1) & 1][ks] = cur[BM * 8 + slot(wn0 + (J + 1) * 16 + (lane & 15), ks * 4 + (lane >> 4))];
+            }
+            if constexpr (J >= 2 && J % 2 == 0) now.template finish<J / 2 - 1>(nxt + BM * 8, v);
+            if constexpr (J % 2 == 0) now.template lookup<J / 2>(lcode, v);
+            if constexpr (J == 1) la.commit(nxt, nullptr, nullptr, 0.f);
+            if constexpr (J == FN - 1) now.template finish<FN / 2 - 1>(nxt + BM * 8, v);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int i = 0; i < FM; ++i) acc[i][J] = mfma16x16x32(af[ks][i], bf[J & 1][ks], acc[i][J]);
+            __builtin_amdgcn_sched_barrier(0);
+            packed_column<J + 1>(la, now, cur, nxt, af, bf, v, acc, lcode, lane, wn0);
+        }
+    }
+    __device__ __forceinline__ static void packed_step(LA &la, LB &lb, const uint4 *cur, uint4 *nxt, int64_t knext,
+                                                       f32x4 (&acc)[FM][FN], const float *lcode, const float *lcode2,
+                                                       float off_b, int lane, int wm0, int wn0) {
+        static_assert(FN == 2 * LB::kPieces, "one piece per two columns");
+        uint4 af[KS][FM], bf[2][KS];
+        float v[8];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int i = 0; i < FM; ++i) af[ks][i] = cur[slot(wm0 + i * 16 + (lane & 15), ks * 4 + (lane >> 4))];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) bf[0][ks] = cur[BM * 8 + slot(wn0 + (lane & 15), ks * 4 + (lane >> 4))];
+        LB now = lb;  // the tile to decode; lb's registers take the one after it
+        now.decode_scales(lcode2, off_b);
+        lb.issue(nxt + BM * 8, knext);
+        __builtin_amdgcn_sched_barrier(0);
+        packed_column<0>(la, now, cur, nxt, af, bf, v, acc, lcode, lane, wn0);
+        la.issue(nxt, knext);
+        __syncthreads();
+    }
+
     __device__ __forceinline__ static void run(const Segment &sg, int64_t m, int64_t n, int64_t m0, int64_t n0,
                                                int64_t tbeg, int64_t tend, f32x4 (&acc)[FM][FN], uint4 *lds0,
                                                uint4 *lds1, const float *lcode, const float *lcode2, int tid,
@@ -693,11 +772,17 @@ struct FastRunner {
         // Step t reads stage (t - tbeg) % 2, which holds tile t; the registers hold tile t+1.
         // Tiles past the end are masked to zeros and never consumed.
         int64_t t = tbeg;
+        const auto one = [&](const uint4 *cur, uint4 *nxt, int64_t knext) {
+            if constexpr (kPacked)
+                packed_step(la, lb, cur, nxt, knext, acc, lcode, lcode2, off_b, lane, wm0, wn0);
+            else
+                step(la, lb, cur, nxt, knext, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+        };
         for (; t + 1 < tend; t += 2) {
-            step(la, lb, lds0, lds1, (t + 2) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
-            step(la, lb, lds1, lds0, (t + 3) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+            one(lds0, lds1, (t + 2) * kBK);
+            one(lds1, lds0, (t + 3) * kBK);
         }
-        if (t < tend) step(la, lb, lds0, lds1, (t + 2) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+        if (t < tend) one(lds0, lds1, (t + 2) * kBK);
     }
 };
 

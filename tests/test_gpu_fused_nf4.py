@@ -74,6 +74,25 @@ def test_fused_forward_and_input_gradient_equal_materialized(m, k, n, r):
             assert norm <= 1e-3, (name, norm)
 
 
+@pytest.mark.parametrize("m,k,n,r", [
+    (66, 64, 72, 8), (128, 128, 256, 8), (251, 192, 520, 24), (255, 4160, 264, 40), (300, 320, 1000, 8),
+    (65, 24576, 520, 256), (257, 8256, 2048, 16), (511, 8192, 776, 72)])
+@pytest.mark.parametrize("nested", [False, True])
+def test_decode_between_the_products_changes_no_bit(m, k, n, r, nested):
+    """65 - 511 rows: the 256 x 256 k-step that spreads the decode over its columns, from one
+    k-tile to 384, odd and even counts, with and without splits, against the dense weight."""
+    packed, state = _weight(n, k, nested=nested, seed=m)
+    dense = materialize(packed, state, torch.bfloat16)
+    x, a, b, _, bias = _inputs(m, k, n, r, seed=n)
+    outs = []
+    for weight, st in ((packed, state), (dense, None)):
+        out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        xa = torch.empty(m, r, device="cuda", dtype=torch.bfloat16)
+        _forward(x, weight, st, a, b, bias, out, xa)
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("blocksize,nested,dtype", [(64, False, torch.bfloat16), (128, True, torch.float32),
                                                     (32, True, torch.bfloat16), (4096, True, torch.bfloat16)])
 def test_fused_state_variants(blocksize, nested, dtype):
