@@ -936,6 +936,24 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     // ------------------------------------------------------------------ epilogue
     if constexpr (B0 == SRC_KT) {
         // KT B fragments leave lane l with columns wn0 + 16 j + (l % 16): element stores.
+        if constexpr (OUT == CT_F32) {
+            // Written transposed, a lane's four rows are consecutive: one 16-byte store each.
+            if (second && p.c1 && p.ldc1 % 4 == 0 && (reinterpret_cast<uintptr_t>(p.c1) & 15) == 0 && !bias_p) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) {
+                    const int64_t row = m0 + wm0 + i * 16 + (lane >> 4) * 4;
+                    if (row >= p.m) continue;  // p.m is a multiple of 8 here (the vector path)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) {
+                        const int64_t col = n0 + wn0 + 16 * j + (lane & 15);
+                        if (col >= ncols) continue;
+                        f32x4 *c = reinterpret_cast<f32x4 *>(p.c1 + col * p.ldc1 + row);
+                        *c = p.beta ? acc[i][j] + *c : acc[i][j];
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
 #pragma unroll
