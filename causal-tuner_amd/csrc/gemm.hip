@@ -1829,22 +1829,48 @@ extern "C" int ct_nf4_fused_supported(const ct_nf4_weight *w) { return nf4_fusab
 
 namespace ct {
 namespace {
-// Rank-r products (narrow outputs: r columns, or up to 1024 for a group's stacked factors;
-// many rows; a reduction of at least 4096): when 128 x 128 tiles give less than one
-// workgroup per CU, the reduction is split 2 to 4 ways (about 512 workgroups, two per CU).
-// Measured on MI355X: at 8192 rows and 256 columns 20-25% faster than 64-wide tiles for
-// reductions of 11008, at 4096 rows 27-40% faster for 8192. Over 2048 the unsplit 64 x 64
-// grid is faster (4096 rows: 12.5 against 20.3 us at 256 columns, 24.9 against 30.7 at
-// 768, 18.7 against 25.4 at 512).
+// Rank-r products: narrow outputs (r columns, or up to 1024 for a group's stacked factors) of
+// more rows than the few-row kernels take. Their output tiles leave most CUs idle, so the
+// reduction is split over workgroups until about 256 to 512 are in flight, each with at least
+// 8 (past 256 workgroups: 16) 64-k tiles, its fp32 partials added in split order; 128 x 128
+// tiles take over where the rows and the reduction are long. Fitted to a sweep on MI355X of
+// 100 - 8192 rows, 16 - 512 columns and reductions of 1024 - 24576, both layouts, over tiles of
+// 64, 128 and 256 with 1 - 32 splits; x a^T, us now (and on the 256 x 256 split or unsplit 64 x
+// 64 grid before): 251 x 256 over 2048 8.2 (19.3), over 24576 19 (28); 1000 x 256 over 4096 12.0
+// (17.5); 4001 x 64 over 4096 13.7 (24.1); 4001 x 256 over 8192 29.0 (47.4); dy b: 251 x 256
+// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 with
+// 64 tiles or more and under 4096 with 128 (a split costs more than it gains: 2000 x 256 over
+// 2048 10.9 unsplit, 12.1 in two), and outputs that fill the grid of 128 x 128 tiles.
+// Wider outputs of up to 256 rows over the longest reductions (the loss's d hidden over its
+// vocabulary) split on 128 x 128 tiles to one workgroup per CU, where the route they took used
+// twice as many splits or 256-row tiles: 128 x 2048 over 49152 52 against 60 us, 128 x 4096 110
+// against 120, 256 x 2048 80 against 87.
 bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
-    if (n > 1024 || m < 4096 || k < 4096) return false;
-    const int64_t tiles = cdiv(m, 128) * cdiv(n, 128);
-    if (tiles >= 256) return false;
-    int64_t s = 512 / tiles;
-    *tile = TILE_128;
-    *splits = (int)(s < 2 ? 2 : (s > 4 ? 4 : s));
-    return true;
+    const int64_t t64 = cdiv(m, 64) * cdiv(n, 64), t128 = cdiv(m, 128) * cdiv(n, 128), kt = cdiv(k, kBK);
+    const auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
+    if (m <= 64 || n <= 0 || t128 >= 256) return false;
+    if (n > 1024) {
+        if (m > 256 || kt < 256 || t128 > 32) return false;
+        *tile = TILE_128;
+        *splits = (int)least(256 / t128, mid_splits(m, n, k));  // the workspace is sized for the latter
+        return *splits > 1;
+    }
+    int64_t s = 1;
+    if ((t64 > 128 && kt >= 64) || (t64 >= 128 && kt >= 128) || (t64 >= 32 && kt >= 256)) {
+        *tile = TILE_128;
+        s = least(least((t128 >= 64 ? 512 : 256) / t128, kt / 16), t128 >= 64 ? 4 : (t128 >= 32 ? 8 : 24));
+    } else {
+        *tile = TILE_64;
+        if (!((t64 >= 64 && kt < 32) || (t64 >= 128 && kt < 64))) {
+            const int64_t deep = least(512 / t64, kt / 16), wide = least(256 / t64, kt / 8);
+            s = least(deep > wide ? deep : wide, 24);
+        }
+    }
+    *splits = (int)(s < 1 ? 1 : s);
+    // Unsplit, only the rows that the 256 x 256 split route would take need the tile named.
+    return s > 1 || m < kMaterializeRows;
 }
+int64_t lowrank_bytes(int64_t m, int64_t n, int splits) { return splits > 1 ? (int64_t)splits * m * n * 4 : 0; }
 }  // namespace
 }  // namespace ct
 
@@ -1852,7 +1878,7 @@ extern "C" int64_t ct_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t tr
                                      int32_t c_dtype) {
     if (trans_a || c_dtype != CT_BF16) return 0;
     int tile, splits;
-    if (lowrank_split(m, n, k, &tile, &splits)) return (int64_t)splits * m * n * 4;
+    if (n <= 1024 && lowrank_split(m, n, k, &tile, &splits)) return lowrank_bytes(m, n, splits);
     const int64_t ks[2] = {k, 0};
     const int sb[2] = {trans_b ? SRC_KC : SRC_KS, trans_b ? SRC_KC : SRC_KS};
     return problem_workspace(m, n, ks, 1, sb);
@@ -1886,10 +1912,12 @@ extern "C" int ct_gemm(const void *a, int64_t lda, int32_t trans_a, const void *
     pr.ws_bytes = workspace ? workspace_bytes : 0;
     pr.vec = vec_ok(pr);
     int tile, splits;
-    if (!bias && c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) && workspace &&
-        workspace_bytes >= (int64_t)splits * m * n * 4) {
+    if (!bias && c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) &&
+        (splits == 1 || workspace) && pr.ws_bytes >= lowrank_bytes(m, n, splits)) {
         pr.tile = tile;
         pr.splits = splits;
+        pr.ws = nullptr;  // unsplit stays unsplit
+        pr.ws_bytes = 0;
         int status = 0;
         const hipError_t e = run_reduction(pr, c, ldc, beta, workspace, workspace_bytes, stream, &status);
         return status ? status : to_status(e);
@@ -2001,6 +2029,30 @@ extern "C" int64_t ct_forward_linear_workspace(int64_t m, int64_t n, int64_t k, 
     const int64_t rest = inner > main ? inner : main;  // the two launches run in order on one stream
     return materialize_kind(nf4, m, n, k + r, kMaterializeRows) ? weight_bytes(n, k) + rest : rest;
 }
+
+// What the static-scratch entry point measures a problem by (ct_forward_linear_static): the
+// decoded weight and the larger of the base product's split partials and of the rank-r product's
+// in its simplest plans. More room only lets ct_gemm pick a faster plan, so a caller near the
+// limit keeps the calls it was given.
+namespace ct {
+int64_t forward_linear_scratch(int64_t m, int64_t n, int64_t k, int64_t r, int32_t nf4) {
+    int64_t inner;
+    const int64_t t128 = cdiv(m, 128) * cdiv(r, 128);
+    if (r > 0 && r <= 1024 && m >= 4096 && k >= 4096 && t128 < 256) {
+        const int64_t s = 512 / t128;
+        inner = (s < 2 ? 2 : (s > 4 ? 4 : s)) * m * r * 4;
+    } else {
+        const int64_t ka[2] = {k, 0};
+        const int sa[2] = {SRC_KC, SRC_KC};
+        inner = problem_workspace(m, r, ka, 1, sa);
+    }
+    const int64_t ks[2] = {k, r};
+    const int sb[2] = {SRC_NF4, SRC_KC};
+    const int64_t main = problem_workspace(m, n, ks, r > 0 ? 2 : 1, sb);
+    const int64_t rest = inner > main ? inner : main;
+    return materialize_kind(nf4, m, n, k + r, kMaterializeRows) ? weight_bytes(n, k) + rest : rest;
+}
+}  // namespace ct
 
 extern "C" int ct_forward_linear(const void *x, int64_t ldx, const void *w_dense, const ct_nf4_weight *w_nf4,
                                  const void *a, const void *b, const void *bias, void *out, int64_t ldo, void *xa,

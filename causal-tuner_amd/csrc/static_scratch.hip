@@ -18,6 +18,10 @@
 
 #include "common.hpp"
 
+namespace ct {
+int64_t forward_linear_scratch(int64_t m, int64_t n, int64_t k, int64_t r, int32_t nf4);  // gemm.hip
+}
+
 static __device__ __align__(256) unsigned char scratch[CT_STATIC_SCRATCH_BYTES];
 
 namespace {
@@ -62,13 +66,16 @@ extern "C" int ct_forward_linear_static(const void *x, int64_t ldx, const void *
     if (m < 0 || n < 0 || k < 0 || r < 0) return -CT_EINVAL_SHAPE;
     if (m == 0 || n == 0) return 0;
     const int32_t kind = w_nf4 ? (w_nf4->nested ? 1 : 2) : 0;
-    const int64_t need = ct_forward_linear_workspace(m, n, k, r, kind);
+    const int64_t need = ct::forward_linear_scratch(m, n, k, r, kind);
     if (need < 0 || need > (int64_t)CT_STATIC_SCRATCH_BYTES) return -CT_EINVAL_WORKSPACE;
+    // The preferred plans may use more (up to the whole array); what does not fit runs unsplit.
+    const int64_t want = ct_forward_linear_workspace(m, n, k, r, kind);
+    const int64_t room = want < (int64_t)CT_STATIC_SCRATCH_BYTES ? want : (int64_t)CT_STATIC_SCRATCH_BYTES;
     void *ws = nullptr;
-    if (need > 0) {
+    if (room > 0) {
         const int st = scratch_address(&ws);
         if (st) return st;
     }
     return ct_forward_linear(x, ldx, w_dense, w_nf4, a, b, bias, out, ldo, xa, ldxa, xa_given, m, n, k, r, epilogue,
-                             ws, need, stream);
+                             ws, room, stream);
 }

@@ -259,3 +259,34 @@ def test_partial_last_round_column_split_in_the_input_gradient():
     want = dy.double() @ w.double() + low @ a.double()
     worst, norm = _err(full, want)
     assert worst <= 8e-3 and norm <= 4e-3, (worst, norm)
+
+
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("m,n,k", [
+    (65, 8, 64), (65, 16, 8192), (251, 256, 2048), (251, 250, 2040), (511, 512, 1024), (513, 72, 4096), (1000, 256, 4096),
+    (4001, 64, 4096), (4001, 256, 8192), (500, 512, 16448),      # rank-r products: every tile and split rule
+    (128, 1216, 16384), (77, 4096, 16448), (256, 2048, 20000),   # up to 256 rows over the longest reductions
+    (513, 1032, 12288), (1000, 2048, 8200)])                     # from 512 rows on 128 x 128 tiles
+def test_planned_products_against_float64(m, n, k, trans_b):
+    """The split plans of narrow and of few-row products (ct_gemm) with and without the
+    workspace they ask for: within one bf16 rounding of float64 (relative norm 2^-9) and
+    bit-identical from call to call."""
+    from causal_tuner.kernels import _native
+    lib = _native.library()
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    b = torch.randn(*((n, k) if trans_b else (k, n)), device="cuda", generator=g).to(torch.bfloat16)
+    want = a.double() @ (b.double().T if trans_b else b.double())
+    need = lib.ct_gemm_workspace(m, n, k, 0, trans_b, _native.CT_BF16)
+    ws = torch.full((max(need, 1),), 255, dtype=torch.uint8, device="cuda")
+
+    def run(pointer, size):
+        out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        status = lib.ct_gemm(a.data_ptr(), k, 0, b.data_ptr(), b.shape[1], trans_b, out.data_ptr(), n, _native.CT_BF16,
+                             None, 0, m, n, k, pointer, size, _native.stream_of(a))
+        assert status == 0
+        return out
+    got, again, alone = run(ws.data_ptr(), need), run(ws.data_ptr(), need), run(None, 0)
+    assert torch.equal(got, again)
+    for out in (got, alone):
+        assert float((out.double() - want).norm() / want.norm()) <= 2 ** -9

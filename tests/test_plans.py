@@ -52,6 +52,23 @@ def test_rank_r_product_splits(m, n, k, splits):
     assert _gemm_ws(m, n, k) == splits * m * n * F32
 
 
+@pytest.mark.parametrize("m,n,k,splits", [
+    (65, 16, 64, 0),           # one k-tile: nothing to split
+    (251, 256, 2048, 4),       # 16 tiles of 64 x 64, 32 k-tiles: 8 per split
+    (251, 256, 24576, 24),     # 64 x 64 tiles, the largest count
+    (500, 512, 1024, 0),       # 64 tiles over 16 k-tiles
+    (500, 512, 24576, 16),     # 128 x 128 tiles: 16 of them to one workgroup per CU
+    (1000, 256, 4096, 4),
+    (1000, 256, 8192, 8),      # past 256 workgroups with 16 k-tiles per split
+    (2000, 256, 2048, 0),
+    (4001, 64, 4096, 4),
+    (4001, 256, 8192, 4),      # 128 x 128 tiles
+    (16384, 256, 6144, 0),     # 256 tiles of 128 x 128 fill the GPU
+])
+def test_rank_r_product_splits_over_rows_and_reductions(m, n, k, splits):
+    assert _gemm_ws(m, n, k) == splits * m * n * F32
+
+
 @pytest.mark.parametrize("m,n,k,trans_b,splits", [
     # few rows: the count (up to one round of resident slots) that spreads the workgroups
     # most evenly over the 256 CUs; rows kernel for trans_b=1, columns kernel for 0

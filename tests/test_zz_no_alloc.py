@@ -69,3 +69,15 @@ def test_static_scratch_refuses_problems_beyond_its_maximum():
     status = lib.ct_forward_linear_static(16, k, None, ctypes.byref(desc), 16, 16, None, 16, n, 16, r, 0, m, n, k, r,
                                           None, None)
     assert status == -5
+
+
+def test_static_scratch_takes_a_weight_that_fills_it():
+    """A decoded weight of exactly the scratch size leaves no room for split partials: the
+    rank-r product then runs unsplit, the projection is still computed."""
+    m, k, n, r = 600, 4096, 8192, 16
+    assert n * k * 2 == _native.CT_STATIC_SCRATCH_BYTES
+    problem = _problem(m, k, n, r, seed=3)
+    got = _run("static", problem, m, k, n, r)
+    want = _run("workspace", problem, m, k, n, r)
+    for g, w in zip(got, want):   # xa sums in another order: one bf16 rounding of it, then of out
+        assert float((g.double() - w.double()).norm() / w.double().norm()) <= 2 ** -8
