@@ -1429,11 +1429,17 @@ bool fast_ok(const Problem &pr) {
     return true;
 }
 
-// Largest tile that still yields about one workgroup per CU (256 CUs).
+// Largest tile that still yields one workgroup per CU (256 CUs), or that the next smaller one
+// cannot replace in one round: the smaller tiles run two workgroups per CU, so past 512 of them
+// a second round costs more than the CUs that the larger tile leaves idle. MI355X, x w^T, us on
+// the larger against the smaller tile: 3421 x 4096 over 4096 (224 tiles of 256, 864 of 128) 94
+// against 122, 5000 x 2048 over 4096 (160, 640) 85 against 93, 1800 x 2048 over 2048 (240 of
+// 128, 928 of 64) 22 against 28, 1200 x 2048 over 2048 (160, 608) 21 against 22; at 512 of the
+// smaller or fewer it wins: 2000 x 4096 over 4096 78 against 67, 1000 x 2048 over 2048 20 against 16.
 int choose_tile(int64_t m, int64_t n, int splits) {
     for (int t = TILE_256; t < TILE_64; ++t) {
-        const int64_t e = kTileEdge[t];
-        if (cdiv(m, e) * cdiv(n, e) * splits >= 256) return t;
+        const int64_t e = kTileEdge[t], f = kTileEdge[t + 1];
+        if (cdiv(m, e) * cdiv(n, e) * splits >= 256 || cdiv(m, f) * cdiv(n, f) * splits > 512) return t;
     }
     return TILE_64;
 }

@@ -290,3 +290,24 @@ def test_planned_products_against_float64(m, n, k, trans_b):
     assert torch.equal(got, again)
     for out in (got, alone):
         assert float((out.double() - want).norm() / want.norm()) <= 2 ** -9
+
+
+@pytest.mark.parametrize("m,n,k", [(2400, 4096, 128), (3421, 2112, 72), (1800, 2048, 200), (1200, 1088, 64)])
+def test_tile_choice_does_not_change_a_result(m, n, k):
+    """Sizes whose grid of large tiles is kept because the next smaller one would need a second
+    round: every element is the same in-order sum on any tile, so rows computed alone (on
+    smaller tiles) are bit-identical."""
+    from causal_tuner.kernels import _native
+    lib = _native.library()
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    b = torch.randn(n, k, device="cuda", generator=g).to(torch.bfloat16)
+
+    def run(rows):
+        out = torch.full((len(rows), n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        assert lib.ct_gemm(rows.data_ptr(), k, 0, b.data_ptr(), k, 1, out.data_ptr(), n, _native.CT_BF16, None, 0,
+                           len(rows), n, k, None, 0, _native.stream_of(a)) == 0
+        return out
+    whole = run(a)
+    for first in (0, 512, (m - 100) // 8 * 8):
+        assert torch.equal(whole[first:first + 100], run(a[first:first + 100].contiguous()))
