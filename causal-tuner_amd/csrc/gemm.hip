@@ -1345,10 +1345,25 @@ constexpr int64_t kLongReduction = 8192;
 // than the split; 6-9% slower at 2048-4096 rows, 2048 columns and 8448); shorter
 // reductions there pay too much for the partials' traffic (2048: 25% slower split). The
 // split count depends only on the shapes.
+// From kMaterializeRows rows on (every weight is dense there), over reductions under 16384,
+// outputs of at most 128 tiles of 128 x 128 split on those, four ways or to one workgroup per
+// CU: fewer, larger partials than 256 x 256 tiles need to fill the GPU (MI355X, over 8192: 512 x
+// 2048 30 against 43 us, 1000 x 2048 45 against 53; at 256 tiles, 2000 x 2048, 76 against 77).
+bool mid_small(int64_t m, int64_t n, int64_t ktot) {
+    return m >= kMaterializeRows && ktot < 16384 && cdiv(m, 128) * cdiv(n, 128) <= 128;
+}
 int mid_splits(int64_t m, int64_t n, int64_t ktot) {
     if (m <= 64 || n <= 0) return 1;
     const int64_t tiles = cdiv(m, 256) * cdiv(n, 256);
     if (m >= kMaterializeRows && (ktot < kLongReduction || tiles >= 256)) return 1;
+    if (mid_small(m, n, ktot)) {
+        const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
+        int64_t s = 256 / t128;
+        if (s < 4) s = 4;
+        const int64_t cap = cdiv(ktot, kBK) / 8;
+        if (s > cap) s = cap;
+        return (int)(s > 32 ? 32 : (s < 1 ? 1 : s));
+    }
     // One round of the one-per-CU 256 x 256 workgroups: a partial second round would
     // take as long as the first.
     int64_t s = 256 / tiles;
@@ -1612,7 +1627,8 @@ hipError_t run(Problem &pr, hipStream_t s) {
         // keep the 256 x 256 runner, the only one with a fused NF4 loader for fp32 partials.
         const bool packed = is_nf4_host(pr.src[0]) || is_nf4_host(pr.src[1]) || is_nf4_host(pr.src[2]) ||
                             is_nf4_host(pr.src[3]);
-        q.tile = (p.m <= 128 && !packed) ? TILE_128 : TILE_256;
+        const int64_t ktot = p.seg[0].k + (p.nseg > 1 ? p.seg[1].k : 0);
+        q.tile = ((p.m <= 128 && !packed) || mid_small(p.m, p.n, ktot)) ? TILE_128 : TILE_256;
         q.ws = nullptr;
         q.ws_bytes = 0;
         q.p.c = pr.ws;

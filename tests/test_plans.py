@@ -69,6 +69,14 @@ def test_rank_r_product_splits_over_rows_and_reductions(m, n, k, splits):
     assert _gemm_ws(m, n, k) == splits * m * n * F32
 
 
+@pytest.mark.parametrize("m,n,k,splits", [
+    (512, 2048, 8192, 4), (1000, 2048, 11008, 4), (513, 1032, 12288, 5),   # at most 128 tiles of 128 x 128
+    (2000, 2048, 8192, 4),     # 256 of them: the 256 x 256 route
+])
+def test_long_reductions_into_small_outputs(m, n, k, splits):
+    assert _gemm_ws(m, n, k) == splits * m * n * F32
+
+
 @pytest.mark.parametrize("m,n,k,trans_b,splits", [
     # few rows: the count (up to one round of resident slots) that spreads the workgroups
     # most evenly over the 256 CUs; rows kernel for trans_b=1, columns kernel for 0
