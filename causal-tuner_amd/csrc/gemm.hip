@@ -849,13 +849,23 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     const int lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave % WAVES_M) * WM, wn0 = (wave / WAVES_M) * WN;
 
-    // Tile order: contiguous ranges per XCD, M-grouped inside a range.
+    // Tile order: contiguous ranges per XCD, M-grouped inside a range. From one split per XCD on
+    // the ranges run over (split, tile), so that an XCD reads its splits' slices of the operands
+    // and no other; taken tile by tile with every split, each of them read the narrow operand in
+    // full, and the fabric was the bound (MI355X: 128 x 2048 over 49152 in 16 splits, 201 MB of w
+    // and 12.6 MB of x, 47 -> 42 us, in 32 53 -> 40; 248 x 256 over 24576 in 24 14.4 -> 10.8).
+    // With fewer splits an XCD holds a share of one either way: the same or slower (MLP at 4001
+    // tokens, 2 to 6 splits: 1274 us, 1283). Workgroups go to the XCDs in linear order.
     const int tiles = p.tiles_m * p.tiles_n;
-    const int pid = blockIdx.x;
+    const bool by_split = gridDim.z >= kXcds;
+    const int count = by_split ? tiles * (int)gridDim.z : tiles;
+    const int pid = (by_split ? (int)blockIdx.z * tiles : 0) + (int)blockIdx.x;
     const int xcd = pid % kXcds, local = pid / kXcds;
-    const int per = (tiles + kXcds - 1) / kXcds;
-    const int tall = tiles % kXcds == 0 ? kXcds : tiles % kXcds;
-    const int rid = xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int per = (count + kXcds - 1) / kXcds;
+    const int tall = count % kXcds == 0 ? kXcds : count % kXcds;
+    const int lin = xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int split = by_split ? lin / tiles : (int)blockIdx.z;
+    const int rid = by_split ? lin % tiles : lin;
     const int group = rid / (kGroupM * p.tiles_n);
     const int first_m = group * kGroupM;
     const int gsize = p.tiles_m - first_m < kGroupM ? p.tiles_m - first_m : kGroupM;
@@ -912,7 +922,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
 
     const int64_t t0 = cdiv(sg0.k, kBK);
     const int64_t t1 = p.nseg > 1 ? cdiv(p.seg[1].k, kBK) : 0;
-    const int64_t tbeg = (int64_t)blockIdx.z * p.tiles_per_split;
+    const int64_t tbeg = (int64_t)split * p.tiles_per_split;
     const int64_t tend = tbeg + p.tiles_per_split < t0 + t1 ? tbeg + p.tiles_per_split : t0 + t1;
     {
         const int64_t b = tbeg, e = tend < t0 ? tend : t0;
@@ -968,7 +978,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
                     const float v = acc[i][j][e] + bias;
                     if constexpr (OUT == CT_F32) {
                         float *c = (second && p.c1) ? p.c1 + col * p.ldc1 + row
-                                                    : static_cast<float *>(p.c) + (int64_t)blockIdx.z * p.split_stride +
+                                                    : static_cast<float *>(p.c) + (int64_t)split * p.split_stride +
                                                           row * p.ldc + out_shift + col;
                         *c = p.beta ? v + *c : v;
                     } else {
@@ -1042,7 +1052,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
 #pragma unroll
             for (int j = 0; j < FN; ++j) v[j] = acc[i][j][e] + bias[j];
             if constexpr (OUT == CT_F32) {
-                float *c = static_cast<float *>(cout) + (int64_t)blockIdx.z * p.split_stride + row * ldc +
+                float *c = static_cast<float *>(cout) + (int64_t)split * p.split_stride + row * ldc +
                            out_shift + col;
                 if (VEC && full && FN % 4 == 0) {
 #pragma unroll
