@@ -649,7 +649,8 @@ struct SchedPattern {
     }
 };
 
-template <int BM, int BN, int SA, int SB, int WAVES_M, int WAVES_N>
+// DEEP keeps two register sets, so two k-tiles' loads are in flight at a time.
+template <int BM, int BN, int SA, int SB, int WAVES_M, int WAVES_N, bool DEEP = false>
 struct FastRunner {
     static constexpr int THREADS = 64 * WAVES_M * WAVES_N;
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
@@ -762,6 +763,27 @@ struct FastRunner {
         const float off_a = is_nf4<SA>() ? *sg.a.offset : 0.f;
         const float off_b = is_nf4<SB>() ? *sg.b.offset : 0.f;
         __syncthreads();  // every wave is done with the buffers of a previous segment
+        if constexpr (DEEP) {
+            // Step t reads stage (t - tbeg) % 2; one register set holds tile t+1, the other t+2.
+            LA la1 = la;
+            LB lb1 = lb;
+            la.issue(lds0, tbeg * kBK);
+            lb.issue(lds0 + BM * 8, tbeg * kBK);
+            la1.issue(lds1, (tbeg + 1) * kBK);
+            lb1.issue(lds1 + BM * 8, (tbeg + 1) * kBK);
+            la.commit(lds0, lcode, lcode2, off_a);
+            lb.commit(lds0 + BM * 8, lcode, lcode2, off_b);
+            la.issue(lds0, (tbeg + 2) * kBK);
+            lb.issue(lds0 + BM * 8, (tbeg + 2) * kBK);
+            __syncthreads();
+            int64_t t = tbeg;
+            for (; t + 1 < tend; t += 2) {
+                step(la1, lb1, lds0, lds1, (t + 3) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+                step(la, lb, lds1, lds0, (t + 4) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+            }
+            if (t < tend) step(la1, lb1, lds0, lds1, (t + 3) * kBK, acc, lcode, lcode2, off_a, off_b, lane, wm0, wn0);
+            return;
+        }
         la.issue(lds0, tbeg * kBK);
         lb.issue(lds0 + BM * 8, tbeg * kBK);
         la.commit(lds0, lcode, lcode2, off_a);
@@ -833,7 +855,8 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams &p, const uint16_
     }
 }
 
-template <int BM, int BN, int A0, int B0, int A1, int B1, int MODE, int OUT, int WAVES_M = 2, int WAVES_N = 2>
+template <int BM, int BN, int A0, int B0, int A1, int B1, int MODE, int OUT, int WAVES_M = 2, int WAVES_N = 2,
+          bool DEEP = false>
 __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     constexpr bool VEC = MODE != 0;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
@@ -927,8 +950,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     {
         const int64_t b = tbeg, e = tend < t0 ? tend : t0;
         if constexpr (MODE == 2)
-            FastRunner<BM, BN, A0, B0, WAVES_M, WAVES_N>::run(sg0, p.m, ncols, m0, n0, b, e, acc, lds0, lds1,
-                                                              lcode, lcode2, tid, wm0, wn0);
+            FastRunner<BM, BN, A0, B0, WAVES_M, WAVES_N, DEEP>::run(sg0, p.m, ncols, m0, n0, b, e, acc, lds0, lds1,
+                                                                    lcode, lcode2, tid, wm0, wn0);
         else
             SegmentRunner<BM, BN, A0, B0, VEC>::run(sg0, p.m, ncols, m0, n0, b, e, acc, lds0, lds1, lcode,
                                                     lcode2, tid, wm0, wn0);
@@ -936,8 +959,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     if (t1 > 0) {
         const int64_t b = tbeg > t0 ? tbeg - t0 : 0, e = tend - t0;
         if constexpr (MODE == 2)
-            FastRunner<BM, BN, A1, B1, WAVES_M, WAVES_N>::run(sg1, p.m, p.n, m0, n0, b, e, acc, lds0, lds1,
-                                                              lcode, lcode2, tid, wm0, wn0);
+            FastRunner<BM, BN, A1, B1, WAVES_M, WAVES_N, DEEP>::run(sg1, p.m, p.n, m0, n0, b, e, acc, lds0, lds1,
+                                                                    lcode, lcode2, tid, wm0, wn0);
         else
             SegmentRunner<BM, BN, A1, B1, VEC>::run(sg1, p.m, p.n, m0, n0, b, e, acc, lds0, lds1, lcode,
                                                     lcode2, tid, wm0, wn0);
@@ -1116,9 +1139,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     gemm_body<256, 256, A0, B0, A1, B1, MODE, OUT>(p);
 }
 
-template <int BM, int BN, int A0, int B0, int A1, int B1, int MODE, int OUT>
+template <int BM, int BN, int A0, int B0, int A1, int B1, int MODE, int OUT, bool DEEP = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_small(const GemmParams p) {
-    gemm_body<BM, BN, A0, B0, A1, B1, MODE, OUT>(p);
+    gemm_body<BM, BN, A0, B0, A1, B1, MODE, OUT, 2, 2, DEEP>(p);
 }
 
 // 256x256 tiles, 8 waves (two per SIMD) of 64x128: each wave's accumulators fit in 128
@@ -1476,6 +1499,21 @@ hipError_t launch_cfg(const GemmParams &p0, int tile, int splits, hipStream_t s)
     p.tiles_m = (int)cdiv(p.m, e);
     p.tiles_n = (int)(p.group_tiles > 0 ? p.group_tiles + cdiv(p.n1, e) : cdiv(p.n, e));
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)splits);
+    // One workgroup per CU has no second one to run while its loads are out. With B read along
+    // its rows (dy b, the loss's d hidden) a second register set covers part of that; at two
+    // workgroups per CU it only costs registers, and KC operands gained nothing. MI355X, one set
+    // and two: 128 x 2048 over 49152 in 16 splits 41.9 and 37.9 us, 4000 x 256 over 8192 in four
+    // 30.4 and 28.0, 4000 x 256 over 2048 on 252 tiles of 64 15.1 and 13.1; past 256 workgroups,
+    // 8192 x 256 over 4096 in four, 28.5 and 29.3.
+    if constexpr (MODE == 2 && A0 == SRC_KC && B0 == SRC_KS && A1 == SRC_KC && B1 == SRC_KS) {
+        if (tile != TILE_256 && (int64_t)grid.x * splits <= 256) {
+            if (tile == TILE_128)
+                gemm_small<128, 128, A0, B0, A1, B1, MODE, OUT, true><<<grid, dim3(kThreads), 0, s>>>(p);
+            else
+                gemm_small<64, 64, A0, B0, A1, B1, MODE, OUT, true><<<grid, dim3(kThreads), 0, s>>>(p);
+            return hipGetLastError();
+        }
+    }
     if (tile == TILE_256 && MODE == 2) gemm_big8<A0, B0, A1, B1, OUT><<<grid, dim3(512), 0, s>>>(p);
     else if (tile == TILE_256) gemm_big<A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
     else if (tile == TILE_128) gemm_small<128, 128, A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
