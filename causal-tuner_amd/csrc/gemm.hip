@@ -1908,8 +1908,9 @@ namespace {
 // 64, 128 and 256 with 1 - 32 splits; x a^T, us now (and on the 256 x 256 split or unsplit 64 x
 // 64 grid before): 251 x 256 over 2048 8.2 (19.3), over 24576 19 (28); 1000 x 256 over 4096 12.0
 // (17.5); 4001 x 64 over 4096 13.7 (24.1); 4001 x 256 over 8192 29.0 (47.4); dy b: 251 x 256
-// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 with
-// 64 tiles or more and under 4096 with 128 (a split costs more than it gains: 2000 x 256 over
+// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 from
+// kMaterializeRows rows on (a second launch for at most two parts, in steps that the host
+// bounds) or with 64 tiles or more, and under 4096 with 128 (a split costs more than it gains: 2000 x 256 over
 // 2048 10.9 unsplit, 12.1 in two), and outputs that fill the grid of 128 x 128 tiles.
 // Wider outputs of up to 256 rows over the longest reductions (the loss's d hidden over its
 // vocabulary) split on 128 x 128 tiles to one workgroup per CU, where the route they took used
@@ -1918,7 +1919,7 @@ namespace {
 bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
     const int64_t t64 = cdiv(m, 64) * cdiv(n, 64), t128 = cdiv(m, 128) * cdiv(n, 128), kt = cdiv(k, kBK);
     const auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
-    if (m <= 64 || n <= 0 || t128 >= 256) return false;
+    if (m <= 64 || n <= 0 || t128 >= 256 || (m >= kMaterializeRows && kt < 32)) return false;
     if (n > 1024) {
         if (m > 256 || kt < 256 || t128 > 32) return false;
         *tile = TILE_128;
