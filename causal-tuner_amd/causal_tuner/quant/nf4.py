@@ -154,9 +154,13 @@ def _device_tables(device):
     """(NF4 midpoints, NF4 code book, dynamic map) on `device`, made once: building the map on
     the host and three copies that wait for it cost more than quantizing a 45 M element weight
     (184 against 33 us for a 64 x 64 weight on an MI355X box). Only read; a state gets copies of
-    its own."""
+    its own. Every table is computed on the host, also under another default device: a copy
+    from the host is complete when it returns, so the tables may be read on any stream, which
+    values computed on the first caller's stream may not."""
+    with torch.inference_mode(False), torch.device("cpu"):
+        host = nf4_thresholds(), nf4_code(), dynamic_map()
     with torch.inference_mode(False):
-        return nf4_thresholds(device), nf4_code(device), dynamic_map().to(device)
+        return tuple(table.to(device) for table in host)
 
 
 def _quantize_nf4_device(weight, blocksize, compress_statistics):
