@@ -38,14 +38,15 @@ struct F32Args {
     const float *a, *b, *bias;
     float *c;
     int64_t lda, ldb, ldc, m, n, k;
-    int tiles_m, tiles_n, beta, vec_c;
+    int tiles_m, tiles_n, beta, vec_a, vec_b, vec_c;
 };
 
 // One operand's tile of a stage of KD * 32 reduction indices, ROWS rows, moved in 16-byte
 // chunks that keep the stored order: KFAST, stored [rows, k], goes to [KD][ROWS][32 k] with
 // tile row n at LDS row frag_row<FRAG>(n); otherwise stored [k, rows], it goes to
-// [k][ROWS], columns XORed with shift(k). VEC: 16-byte loads (aligned base, pitch and
-// contiguous extent in multiples of 4).
+// [k][ROWS], columns XORed with shift(k). VEC: every chunk is one 16-byte load or none of it
+// (aligned base, pitch and contiguous extent in multiples of 4). Otherwise `vec` says whether
+// whole chunks may be loaded so; the rest go element by element.
 template <int ROWS, int KD, int THREADS, bool KFAST, bool VEC, int FRAG>
 struct Tile {
     static constexpr int kPer = ROWS * 8 * KD / THREADS;
@@ -67,7 +68,7 @@ struct Tile {
         }
     }
     __device__ __forceinline__ void load(const float *p, int64_t ld, int64_t r0, int64_t rows, int64_t k0,
-                                         int64_t kdim, int tid) {
+                                         int64_t kdim, bool vec, int tid) {
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             int row, kk;
@@ -77,6 +78,8 @@ struct Tile {
             const float *src = KFAST ? p + rg * ld + kg : p + kg * ld + rg;
             if constexpr (VEC) {
                 v[i] = left > 0 ? *reinterpret_cast<const f32x4 *>(src) : f32x4{0.f, 0.f, 0.f, 0.f};
+            } else if (vec && left >= 4) {
+                v[i] = *reinterpret_cast<const f32x4 *>(src);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[i][j] = j < left ? src[j] : 0.f;
@@ -185,8 +188,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KW) __attribute__((amdgpu_
     TileB lb[SETS];
     const int64_t steps = (g.k + kDepth - 1) / kDepth;
     const auto load = [&](auto set, int64_t s) {
-        la[set].load(g.a, g.lda, m0, g.m, s * kDepth, g.k, tid);
-        lb[set].load(g.b, g.ldb, n0, g.n, s * kDepth, g.k, tid);
+        la[set].load(g.a, g.lda, m0, g.m, s * kDepth, g.k, g.vec_a, tid);
+        lb[set].load(g.b, g.ldb, n0, g.n, s * kDepth, g.k, g.vec_b, tid);
     };
     const auto store = [&](auto set, int stage) {
         la[set].store(lds + stage * kStage, tid);
@@ -293,10 +296,8 @@ void launch_vec(Shape shape, bool vec, const F32Args &g, hipStream_t s) {
     else launch_shape<AK, BKF, false>(shape, g, s);
 }
 
-// 16-byte loads: aligned base, pitch and extent of the contiguous dimension in multiples of 4.
-bool operand_vec(const float *p, int64_t ld, int64_t contiguous) {
-    return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && contiguous % 4 == 0;
-}
+// 16-byte loads of an operand's whole chunks: aligned base and pitch in multiples of 4.
+bool operand_vec(const float *p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; }
 
 }  // namespace
 }  // namespace ct
@@ -320,7 +321,10 @@ extern "C" int ct_gemm_f32(const float *a, int64_t lda, int32_t trans_a, const f
     if (tm * tn > 0x7fffffff) return -CT_EINVAL_SHAPE;
     g.tiles_m = (int)tm;
     g.tiles_n = (int)tn;
-    const bool vec = operand_vec(a, lda, acols) && operand_vec(b, ldb, bcols);
+    g.vec_a = operand_vec(a, lda);
+    g.vec_b = operand_vec(b, ldb);
+    // Both operands in whole chunks: the kernels without the per-chunk choice.
+    const bool vec = g.vec_a && g.vec_b && acols % 4 == 0 && bcols % 4 == 0;
     if (trans_a && trans_b) launch_vec<false, true>(shape, vec, g, stream);
     else if (trans_a) launch_vec<false, false>(shape, vec, g, stream);
     else if (trans_b) launch_vec<true, true>(shape, vec, g, stream);

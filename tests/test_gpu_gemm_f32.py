@@ -48,13 +48,14 @@ def test_layouts_against_float64(m, n, k, trans_l, trans_r):
 
 
 @pytest.mark.parametrize("m,n,k", [(1000, 64, 2048), (31, 33, 129), (65, 4, 4095), (1028, 1020, 132), (2049, 2044, 36),
-                                   (33, 1000, 128)])
+                                   (33, 1000, 128), (2049, 2044, 100), (2048, 2052, 260), (2047, 2049, 131)])
 @pytest.mark.parametrize("trans_l", [False, True])
 @pytest.mark.parametrize("trans_r", [False, True])
 def test_every_tile_with_bias_and_accumulation(m, n, k, trans_l, trans_r):
     """The three output tiles (32 x 32 with the reduction split inside the workgroup, 64 x 64,
-    128 x 128) at partial tiles and stages, bias and accumulation in one call sequence, against
-    float64."""
+    128 x 128) at partial tiles and stages (the last tile with two, four, nine and five of its
+    32-k stages: the main loop refills from the third on), bias and accumulation in one call
+    sequence, against float64; a second call repeats the bits."""
     from causal_tuner.kernels.linear import mm_f32
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     left = torch.randn(k, m, device="cuda", generator=g).T if trans_l else torch.randn(m, k, device="cuda", generator=g)
@@ -64,8 +65,41 @@ def test_every_tile_with_bias_and_accumulation(m, n, k, trans_l, trans_r):
     mm_f32(left, right, out, bias=bias)
     want = _ref(left, right, bias=bias)
     _close(out, want, k)
+    again = torch.empty_like(out)
+    mm_f32(left, right, again, bias=bias)
+    assert torch.equal(out, again)
     mm_f32(left, right, out, add=True)
     _close(out, want + _ref(left, right), k)
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 60, 404), (1028, 1020, 132), (2050, 2046, 70)])
+@pytest.mark.parametrize("trans_l", [False, True])
+@pytest.mark.parametrize("trans_r", [False, True])
+def test_alignment_is_judged_per_operand_and_changes_no_bit(m, n, k, trans_l, trans_r):
+    """Each tile with either operand, or both, at an unaligned start, an odd pitch, or a whole
+    pitch around a ragged extent (whole chunks by vector, the rest by element): the sums are
+    those of the aligned, dense operands."""
+    from causal_tuner.kernels.linear import mm_f32
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    stored = [torch.randn(*(shape[::-1] if t else shape), device="cuda", generator=g)
+              for shape, t in (((m, k), trans_l), ((k, n), trans_r))]
+
+    def product(left, right):
+        out = torch.full((m, n), float("nan"), device="cuda")
+        mm_f32(left.T if trans_l else left, right.T if trans_r else right, out)
+        return out
+
+    def placed(t, first, pitch):
+        wide = torch.full((t.shape[0] * pitch + first,), float("nan"), device="cuda")
+        view = wide[first:].view(t.shape[0], pitch)[:, :t.shape[1]]
+        view.copy_(t)
+        return view
+    want = product(*stored)
+    _close(want, _ref(stored[0].T if trans_l else stored[0], stored[1].T if trans_r else stored[1]), k)
+    for first, spare in ((1, 0), (0, 1), (0, None)):   # None: the next multiple of 4 past the extent
+        moved = [placed(t, first, t.shape[1] + (8 - t.shape[1] % 4 if spare is None else spare)) for t in stored]
+        for operands in ((moved[0], stored[1]), (stored[0], moved[1]), moved):
+            assert torch.equal(product(*operands), want), (first, spare)
 
 
 def test_bias_accumulate_and_strided_views():
