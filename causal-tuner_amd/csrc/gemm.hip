@@ -1132,7 +1132,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     }
 }
 
-// 256x256 tiles: one workgroup per CU, 512 registers per lane (accumulators in AGPRs).
+// 256x256 tiles of the generic runner: one workgroup per CU, 512 registers per lane (accumulators
+// in AGPRs).
 template <int A0, int B0, int A1, int B1, int MODE, int OUT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_big(
     const GemmParams p) {
@@ -1514,9 +1515,10 @@ hipError_t launch_cfg(const GemmParams &p0, int tile, int splits, hipStream_t s)
             return hipGetLastError();
         }
     }
-    if (tile == TILE_256 && MODE == 2) gemm_big8<A0, B0, A1, B1, OUT><<<grid, dim3(512), 0, s>>>(p);
-    else if (tile == TILE_256) gemm_big<A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
-    else if (tile == TILE_128) gemm_small<128, 128, A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
+    if (tile == TILE_256) {
+        if constexpr (MODE == 2) gemm_big8<A0, B0, A1, B1, OUT><<<grid, dim3(512), 0, s>>>(p);
+        else gemm_big<A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
+    } else if (tile == TILE_128) gemm_small<128, 128, A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
     else gemm_small<64, 64, A0, B0, A1, B1, MODE, OUT><<<grid, dim3(kThreads), 0, s>>>(p);
     return hipGetLastError();
 }
