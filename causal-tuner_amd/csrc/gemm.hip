@@ -1986,7 +1986,7 @@ extern "C" int ct_gemm(const void *a, int64_t lda, int32_t trans_a, const void *
     pr.vec = vec_ok(pr);
     int tile, splits;
     if (!bias && c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) &&
-        (splits == 1 || workspace) && pr.ws_bytes >= lowrank_bytes(m, n, splits)) {
+        (splits == 1 || (workspace && aligned16(workspace))) && pr.ws_bytes >= lowrank_bytes(m, n, splits)) {
         pr.tile = tile;
         pr.splits = splits;
         pr.ws = nullptr;  // unsplit stays unsplit

@@ -292,6 +292,31 @@ def test_planned_products_against_float64(m, n, k, trans_b):
         assert float((out.double() - want).norm() / want.norm()) <= 2 ** -9
 
 
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(65, 16, 8192), (251, 256, 2048), (4001, 256, 8192), (128, 2048, 16384),
+                                   (300, 2048, 8192)])
+def test_a_workspace_that_is_not_16_byte_aligned_counts_as_absent(m, n, k, trans_b):
+    """The partials' 16-byte stores need an aligned workspace; one that is not is left alone and
+    the product is that of a call without any, bit for bit."""
+    from causal_tuner.kernels import _native
+    lib = _native.library()
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    b = torch.randn(*((n, k) if trans_b else (k, n)), device="cuda", generator=g).to(torch.bfloat16)
+    need = lib.ct_gemm_workspace(m, n, k, 0, trans_b, _native.CT_BF16)
+    assert need > 0
+    ws = torch.full((need + 16,), 77, dtype=torch.uint8, device="cuda")
+
+    def run(pointer, size):
+        out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        assert lib.ct_gemm(a.data_ptr(), k, 0, b.data_ptr(), b.shape[1], trans_b, out.data_ptr(), n, _native.CT_BF16,
+                           None, 0, m, n, k, pointer, size, _native.stream_of(a)) == 0
+        return out
+    got = run(ws.data_ptr() + 8, need)
+    assert torch.equal(got, run(None, 0))
+    assert bool((ws == 77).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(2400, 4096, 128), (3421, 2112, 72), (1800, 2048, 200), (1200, 1088, 64)])
 def test_tile_choice_does_not_change_a_result(m, n, k):
     """Sizes whose grid of large tiles is kept because the next smaller one would need a second
