@@ -1781,7 +1781,7 @@ int64_t split_workspace_bytes(int64_t m, int64_t n, int64_t kred) {
     return s > 1 ? (int64_t)s * m * n * (int64_t)sizeof(float) : 0;
 }
 
-// out (fp32 or bf16) = sum_k A B (+ out), through fixed-order split partials in ws when
+// out (fp32 or bf16) = sum_k A B (+ bias) (+ out), through fixed-order split partials in ws when
 // the output alone cannot fill the GPU.
 hipError_t run_reduction(Problem pr, void *out, int64_t ldo, int add, void *ws, int64_t ws_bytes,
                          hipStream_t s, int *status) {
@@ -1811,15 +1811,15 @@ hipError_t run_reduction(Problem pr, void *out, int64_t ldo, int add, void *ws, 
     p.ldc = p.n;
     p.split_stride = p.m * p.n;
     p.beta = 0;
+    const uint16_t *bias = p.bias;  // added by the reduction
     p.bias = nullptr;
     pr.vec = pr.vec && aligned16(ws) && p.n % 8 == 0;
     hipError_t e = run(pr, s);
     if (e != hipSuccess) return e;
     if (final_out == CT_F32)
-        return launch_reduce<CT_F32>(static_cast<float *>(ws), splits, p.split_stride, p.m, p.n, out, ldo, add,
-                                     nullptr, s);
-    return launch_reduce<CT_BF16>(static_cast<float *>(ws), splits, p.split_stride, p.m, p.n, out, ldo, add, nullptr,
-                                  s);
+        return launch_reduce<CT_F32>(static_cast<float *>(ws), splits, p.split_stride, p.m, p.n, out, ldo, add, bias,
+                                     s);
+    return launch_reduce<CT_BF16>(static_cast<float *>(ws), splits, p.split_stride, p.m, p.n, out, ldo, add, bias, s);
 }
 
 int to_status(hipError_t e) { return e == hipSuccess ? 0 : (int)e; }
@@ -1985,7 +1985,7 @@ extern "C" int ct_gemm(const void *a, int64_t lda, int32_t trans_a, const void *
     pr.ws_bytes = workspace ? workspace_bytes : 0;
     pr.vec = vec_ok(pr);
     int tile, splits;
-    if (!bias && c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) &&
+    if (c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) &&
         (splits == 1 || (workspace && aligned16(workspace))) && pr.ws_bytes >= lowrank_bytes(m, n, splits)) {
         pr.tile = tile;
         pr.splits = splits;

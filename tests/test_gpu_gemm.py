@@ -293,6 +293,33 @@ def test_planned_products_against_float64(m, n, k, trans_b):
 
 
 @pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(128, 64, 24576), (251, 256, 2048), (251, 250, 2040), (400, 512, 1024), (1000, 1024, 8192),
+                                   (4001, 256, 8192), (128, 2048, 16384)])
+def test_biased_products_take_the_plan_their_workspace_is_sized_for(m, n, k, trans_b):
+    """A bias does not change the plan: where the workspace query asks for partials they are
+    written, and bias and existing output are added once, within one bf16 rounding of float64
+    (relative norm 2^-9)."""
+    from causal_tuner.kernels import _native
+    lib = _native.library()
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    b = torch.randn(*((n, k) if trans_b else (k, n)), device="cuda", generator=g).to(torch.bfloat16)
+    bias = (torch.randn(n + 1, device="cuda", generator=g) * 30).to(torch.bfloat16)
+    start = (torch.randn(m, n, device="cuda", generator=g) * 30).to(torch.bfloat16)
+    product = a.double() @ (b.double().T if trans_b else b.double())
+    need = lib.ct_gemm_workspace(m, n, k, 0, trans_b, _native.CT_BF16)
+    for first, beta in ((0, 0), (0, 1), (1, 0)):   # an unaligned bias takes the element-wise sums
+        ws = torch.full((max(need, 1),), 255, dtype=torch.uint8, device="cuda")
+        out = start.clone()
+        added = bias[first:first + n]
+        assert lib.ct_gemm(a.data_ptr(), k, 0, b.data_ptr(), b.shape[1], trans_b, out.data_ptr(), n, _native.CT_BF16,
+                           added.data_ptr(), beta, m, n, k, ws.data_ptr(), need, _native.stream_of(a)) == 0
+        want = product + added.double() + (start.double() if beta else 0)
+        assert float((out.double() - want).norm() / want.norm()) <= 2 ** -9
+        assert need == 0 or bool((ws != 255).any())
+
+
+@pytest.mark.parametrize("trans_b", [0, 1])
 @pytest.mark.parametrize("m,n,k", [(65, 16, 8192), (251, 256, 2048), (4001, 256, 8192), (128, 2048, 16384),
                                    (300, 2048, 8192)])
 def test_a_workspace_that_is_not_16_byte_aligned_counts_as_absent(m, n, k, trans_b):
