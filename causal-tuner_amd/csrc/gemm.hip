@@ -1478,6 +1478,10 @@ bool fast_ok(const Problem &pr) {
     return true;
 }
 
+int64_t total_tiles(const GemmParams &p) {
+    return cdiv(p.seg[0].k, kBK) + (p.nseg > 1 ? cdiv(p.seg[1].k, kBK) : 0);
+}
+
 // Largest tile that still yields one workgroup per CU (256 CUs), or that the next smaller one
 // cannot replace in one round: the smaller tiles run two workgroups per CU, so past 512 of them
 // a second round costs more than the CUs that the larger tile leaves idle. MI355X, x w^T, us on
@@ -1485,10 +1489,26 @@ bool fast_ok(const Problem &pr) {
 // against 122, 5000 x 2048 over 4096 (160, 640) 85 against 93, 1800 x 2048 over 2048 (240 of
 // 128, 928 of 64) 22 against 28, 1200 x 2048 over 2048 (160, 608) 21 against 22; at 512 of the
 // smaller or fewer it wins: 2000 x 4096 over 4096 78 against 67, 1000 x 2048 over 2048 20 against 16.
-int choose_tile(int64_t m, int64_t n, int splits) {
+// A second round costs its reduction, and the fewer, larger workgroups give up the overlap of
+// one's epilogue with another's products, so the rule waits for a reduction of at least:
+//   128 over 64: 24 k-tiles (mean of 22 sizes, larger / smaller tile: 1.04 at 512, 0.95 and up
+//     to 1.04 at 1024, 0.92 at 1536, 0.87 from 2048); 64 with SiLU or RoPE inside (8 sizes: RoPE
+//     1.21 at 1024, 1.07 at 2048, 0.95 at 4096; SiLU 1.14, 1.01, 0.91);
+//   256 over 128: any (0.85 at 512, 0.83 at 2048; the SiLU steps become a pass of their own
+//     there, 0.82 - 0.96; RoPE 0.93, 0.89); 24 with a residual (1.05 at 1024, 0.99 at 1536, 0.91
+//     at 2048) over a dense weight. A packed one is decoded again in every tile row: any (257 -
+//     511 rows of 16640 - 28672 columns 0.61 - 0.79, with a residual at most 0.89).
+int64_t second_round_from(const Problem &pr, int tile) {
+    const int kind = pr.p.epi.kind;
+    if (tile == TILE_128) return kind == CT_EPI_SILU || kind == CT_EPI_ROPE ? 64 : 24;
+    return kind == CT_EPI_RESIDUAL && !is_nf4_host(pr.src[1]) ? 24 : 0;
+}
+int choose_tile(const Problem &pr) {
+    const GemmParams &p = pr.p;
     for (int t = TILE_256; t < TILE_64; ++t) {
         const int64_t e = kTileEdge[t], f = kTileEdge[t + 1];
-        if (cdiv(m, e) * cdiv(n, e) * splits >= 256 || cdiv(m, f) * cdiv(n, f) * splits > 512) return t;
+        if (cdiv(p.m, e) * cdiv(p.n, e) * pr.splits >= 256) return t;
+        if (cdiv(p.m, f) * cdiv(p.n, f) * pr.splits > 512 && total_tiles(p) >= second_round_from(pr, t)) return t;
     }
     return TILE_64;
 }
@@ -1547,10 +1567,6 @@ template <int A0, int B0, int A1, int B1>
 hipError_t launch_vec_out(const Problem &pr, int tile, hipStream_t s) {
     return pr.out == CT_F32 ? launch_mode<A0, B0, A1, B1, CT_F32>(pr, tile, s)
                             : launch_mode<A0, B0, A1, B1, CT_BF16>(pr, tile, s);
-}
-
-int64_t total_tiles(const GemmParams &p) {
-    return cdiv(p.seg[0].k, kBK) + (p.nseg > 1 ? cdiv(p.seg[1].k, kBK) : 0);
 }
 
 #define CT_LAYOUT(a0, b0, a1, b1) \
@@ -1612,7 +1628,7 @@ bool epilogue_fused(const Problem &pr) {
         const int sb[2] = {pr.src[1], p.nseg > 1 ? pr.src[3] : pr.src[1]};
         if (skinny_supported(p, sa, sb, pr.out)) return false;
     }
-    const int tile = pr.tile >= 0 ? pr.tile : choose_tile(p.m, p.n, pr.splits);
+    const int tile = pr.tile >= 0 ? pr.tile : choose_tile(pr);
     return !(tile == TILE_256 && (p.epi.kind == CT_EPI_SILU || p.epi.kind == CT_EPI_DSILU));
 }
 
@@ -1701,7 +1717,7 @@ hipError_t run(Problem &pr, hipStream_t s) {
             if (e != hipErrorNotSupported) return e;
         }
     }
-    const int tile = pr.tile >= 0 ? pr.tile : choose_tile(p.m, p.n, pr.splits);
+    const int tile = pr.tile >= 0 ? pr.tile : choose_tile(pr);
     if (pr.tile < 0 && tile == TILE_256) {
         int64_t head = 0;
         if (column_split(pr, &head)) {
@@ -2262,7 +2278,7 @@ extern "C" int ct_group_forward(const void *x, int64_t ldx, int32_t count, const
     pr.splits = 1;
     // The tile the whole output would take, or the largest smaller one on whose edge the
     // second projection starts.
-    int tile = choose_tile(m, nt, 1);
+    int tile = choose_tile(pr);
     while (tile < TILE_64 && n[0] % kTileEdge[tile]) ++tile;
     pr.tile = tile;
     // Without a workspace the split route is not taken: the tiled kernels only.

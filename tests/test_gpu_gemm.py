@@ -344,11 +344,14 @@ def test_a_workspace_that_is_not_16_byte_aligned_counts_as_absent(m, n, k, trans
     assert bool((ws == 77).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(2400, 4096, 128), (3421, 2112, 72), (1800, 2048, 200), (1200, 1088, 64)])
+@pytest.mark.parametrize("m,n,k", [
+    (2400, 4096, 128), (3421, 2600, 72),      # 160 and 154 tiles of 256 x 256 (608 and 567 of 128)
+    (1800, 2048, 1536), (1210, 2000, 1544),   # 240 and 160 of 128 x 128 (928 and 608 of 64), 24 k-tiles
+    (1800, 2048, 1528)])                      # a k-tile short of that: 64 x 64
 def test_tile_choice_does_not_change_a_result(m, n, k):
     """Sizes whose grid of large tiles is kept because the next smaller one would need a second
-    round: every element is the same in-order sum on any tile, so rows computed alone (on
-    smaller tiles) are bit-identical."""
+    round, and one just short of the rule: every element is the same in-order sum on any tile, so
+    rows computed alone (100 rows give too few tiles for any but 64 x 64) are bit-identical."""
     from causal_tuner.kernels import _native
     lib = _native.library()
     g = torch.Generator(device="cuda").manual_seed(m)
