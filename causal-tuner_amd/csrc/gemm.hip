@@ -872,15 +872,11 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     const int lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave % WAVES_M) * WM, wn0 = (wave / WAVES_M) * WN;
 
-    // Tile order: contiguous ranges per XCD, M-grouped inside a range. From one split per XCD on
-    // the ranges run over (split, tile), so that an XCD reads its splits' slices of the operands
-    // and no other; taken tile by tile with every split, each of them read the narrow operand in
-    // full, and the fabric was the bound (MI355X: 128 x 2048 over 49152 in 16 splits, 201 MB of w
-    // and 12.6 MB of x, 47 -> 42 us, in 32 53 -> 40; 248 x 256 over 24576 in 24 14.4 -> 10.8).
-    // With fewer splits an XCD holds a share of one either way: the same or slower (MLP at 4001
-    // tokens, 2 to 6 splits: 1274 us, 1283). Workgroups go to the XCDs in linear order.
+    // Tile order: contiguous ranges per XCD, M-grouped inside a range. With by_split (see
+    // splits_by_xcd) the ranges run over (split, tile), so that an XCD reads its splits' slices of
+    // the operands and no other. Workgroups go to the XCDs in linear order.
     const int tiles = p.tiles_m * p.tiles_n;
-    const bool by_split = gridDim.z >= kXcds;
+    const bool by_split = p.by_split;
     const int count = by_split ? tiles * (int)gridDim.z : tiles;
     const int pid = (by_split ? (int)blockIdx.z * tiles : 0) + (int)blockIdx.x;
     const int xcd = pid % kXcds, local = pid / kXcds;
@@ -1513,12 +1509,28 @@ int choose_tile(const Problem &pr) {
     return TILE_64;
 }
 
+// Whether an XCD takes whole splits rather than every split of its tiles. Taken tile by tile,
+// each XCD reads the operands of its tiles over the full reduction, and the fabric is the bound
+// where that is long: 128 x 2048 over 49152 in 16 splits, 201 MB of w and 12.6 MB of x, 47 us
+// against 42 by split, in 32 62.5 against 49; 300 x 256 over 24576 in 18 22.4 against 17.3.
+// Measured on MI355X over 754 plans of 4 - 32 splits, by split / tile by tile: 0.91 in the mean
+// from 16 splits over at least 16384, and 0.95 from 8 on tiles of 128 and 64 with at least two
+// tiles each way (512 x 1024 over 49152 in 8 64 against 82 us). Left tile by tile: shorter
+// reductions (8192: 1.0, up to 1.2; dA/dB of 1000 x 1000 over 8192 tokens 27.7 against 29.7 us),
+// a single row or column of tiles in 8 to 15 splits (nothing is shared: 128 x 8192 over 49152
+// 188 against 204) and the 256 x 256 tile there (200 x 8192 over 24576 115 against 131).
+bool splits_by_xcd(const GemmParams &p, int tile, int splits) {
+    if (total_tiles(p) < 256) return false;
+    return splits >= 2 * kXcds || (splits >= kXcds && tile != TILE_256 && p.tiles_m > 1 && p.tiles_n > 1);
+}
+
 template <int A0, int B0, int A1, int B1, int MODE, int OUT>
 hipError_t launch_cfg(const GemmParams &p0, int tile, int splits, hipStream_t s) {
     GemmParams p = p0;
     const int e = kTileEdge[tile];
     p.tiles_m = (int)cdiv(p.m, e);
     p.tiles_n = (int)(p.group_tiles > 0 ? p.group_tiles + cdiv(p.n1, e) : cdiv(p.n, e));
+    p.by_split = splits_by_xcd(p, tile, splits);
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)splits);
     // One workgroup per CU has no second one to run while its loads are out. With B read along
     // its rows (dy b, the loss's d hidden) a second register set covers part of that; at two
@@ -1550,6 +1562,7 @@ hipError_t launch_cfg_fast(const GemmParams &p0, int splits, hipStream_t s) {
     constexpr int e = TILE == TILE_256 ? 256 : 128;
     p.tiles_m = (int)cdiv(p.m, e);
     p.tiles_n = (int)(p.group_tiles > 0 ? p.group_tiles + cdiv(p.n1, e) : cdiv(p.n, e));
+    p.by_split = splits_by_xcd(p, TILE, splits);
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)splits);
     if constexpr (TILE == TILE_256) gemm_big8<A0, B0, A1, B1, OUT><<<grid, dim3(512), 0, s>>>(p);
     else gemm_small<128, 128, A0, B0, A1, B1, 2, OUT><<<grid, dim3(kThreads), 0, s>>>(p);

@@ -38,6 +38,7 @@ struct GemmParams {
     const uint16_t *bias;     // bf16 [n] or null
     int beta;                 // add the existing C
     int tiles_m, tiles_n;
+    int by_split;             // each XCD takes whole splits (its own range of blockIdx.z)
     const float *code;        // NF4 code book [16]
     const float *code2;       // NF4 second-level code book [256]
     float *split_ws;          // few-row kernels: fp32 split partials [splits][m][n]
