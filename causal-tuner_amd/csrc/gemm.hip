@@ -1939,18 +1939,28 @@ namespace {
 // 64, 128 and 256 with 1 - 32 splits; x a^T, us now (and on the 256 x 256 split or unsplit 64 x
 // 64 grid before): 251 x 256 over 2048 8.2 (19.3), over 24576 19 (28); 1000 x 256 over 4096 12.0
 // (17.5); 4001 x 64 over 4096 13.7 (24.1); 4001 x 256 over 8192 29.0 (47.4); dy b: 251 x 256
-// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 from
-// kMaterializeRows rows on (a second launch for at most two parts, in steps that the host
-// bounds) or with 64 tiles or more, and under 4096 with 128 (a split costs more than it gains: 2000 x 256 over
-// 2048 10.9 unsplit, 12.1 in two), and outputs that fill the grid of 128 x 128 tiles.
+// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 with
+// 64 tiles or more, and under 4096 with 128 (a split costs more than it gains), outputs that fill
+// the grid of 128 x 128 tiles, and what split_repays_launch turns away.
 // Wider outputs of up to 256 rows over the longest reductions (the loss's d hidden over its
 // vocabulary) split on 128 x 128 tiles to one workgroup per CU, where the route they took used
 // twice as many splits or 256-row tiles: 128 x 2048 over 49152 52 against 60 us, 128 x 4096 110
 // against 120, 256 x 2048 80 against 87.
+// A split adds a launch, which costs a step that the host bounds about 4 us per product whatever it
+// saves on the GPU. Below kMaterializeRows the route it replaces splits as well, and so it does
+// from kLongReduction on. Between, a projection (m rows, k x k) occupies the GPU for less time
+// than the host takes to issue it until m k^2 is about 4e10 (250 us), and the product stays
+// unsplit. MI355X, a step with its backward, split against unsplit: 512 rows, 2048 x 2048, rank
+// 16 294 against 283 us (two of 7.5 us for 10.5), 1000 rows, 4096 x 4096, rank 64 297 against 286.
+// Under 4096 the saving (3 to 6 us) never repays it.
+bool split_repays_launch(int64_t m, int64_t k) {
+    if (m < kMaterializeRows || k >= kLongReduction) return true;
+    return k >= 4096 && (double)m * (double)k * (double)k >= 4e10;
+}
 bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
     const int64_t t64 = cdiv(m, 64) * cdiv(n, 64), t128 = cdiv(m, 128) * cdiv(n, 128), kt = cdiv(k, kBK);
     const auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
-    if (m <= 64 || n <= 0 || t128 >= 256 || (m >= kMaterializeRows && kt < 32)) return false;
+    if (m <= 64 || n <= 0 || t128 >= 256 || !split_repays_launch(m, k)) return false;
     if (n > 1024) {
         if (m > 256 || kt < 256 || t128 > 32) return false;
         *tile = TILE_128;

@@ -57,8 +57,14 @@ def test_rank_r_product_splits(m, n, k, splits):
     (251, 256, 2048, 4),       # 16 tiles of 64 x 64, 32 k-tiles: 8 per split
     (251, 256, 24576, 24),     # 64 x 64 tiles, the largest count
     (500, 512, 1024, 0),       # 64 tiles over 16 k-tiles
+    (511, 1024, 2048, 0),      # 128 tiles over 32
     (500, 512, 24576, 16),     # 128 x 128 tiles: 16 of them to one workgroup per CU
-    (1000, 256, 4096, 4),
+    # from 512 rows over less than 8192: split only where the GPU, not the host, bounds a step
+    (512, 16, 2048, 0),
+    (1000, 256, 4096, 0),
+    (2383, 64, 4096, 0),       # m k^2 just under 4e10
+    (2385, 64, 4096, 6),       # and just above
+    (6000, 64, 4032, 0),       # never under 4096
     (1000, 256, 8192, 8),      # past 256 workgroups with 16 k-tiles per split
     (2000, 256, 2048, 0),
     (4001, 64, 4096, 4),
