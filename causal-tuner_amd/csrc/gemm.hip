@@ -1366,6 +1366,11 @@ constexpr int kTileEdge[3] = {256, 128, 64};
 constexpr int64_t kMaterializeRows = CT_MATERIALIZE_ROWS;
 // Reductions at least this long keep the split route from kMaterializeRows rows on.
 constexpr int64_t kLongReduction = 8192;
+// Split count that balances `tiles` (of 128 x 128) over the CUs: up to 64 tiles, splits to one
+// workgroup per CU; past that two per CU, as a count just over 256 leaves some CUs with two
+// workgroups and the rest with one. MI355X, 72 tiles (1030 x 1024 over 24576), us in 3, 4, 6, 7
+// and 8 splits (216 to 576 workgroups): 93, 124, 92, 82, 109; 96 tiles over 8192 in 4 and 5: 50, 46.
+int64_t balanced_splits(int64_t tiles) { return (tiles > 64 ? 512 : 256) / tiles; }
 // Rows between the few-row kernels (m <= 64) and kMaterializeRows, and more rows with a
 // reduction of at least kLongReduction: the output leaves the 256 x 256 grid short of one
 // round, so the fast runner splits the reduction and the fp32 partials are added in split
@@ -1376,9 +1381,9 @@ constexpr int64_t kLongReduction = 8192;
 // reductions there pay too much for the partials' traffic (2048: 25% slower split). The
 // split count depends only on the shapes.
 // From kMaterializeRows rows on (every weight is dense there), over reductions under 16384,
-// outputs of at most 128 tiles of 128 x 128 split on those, four ways or to one workgroup per
-// CU: fewer, larger partials than 256 x 256 tiles need to fill the GPU (MI355X, over 8192: 512 x
-// 2048 30 against 43 us, 1000 x 2048 45 against 53; at 256 tiles, 2000 x 2048, 76 against 77).
+// outputs of at most 128 tiles of 128 x 128 split on those (balanced_splits): fewer, larger
+// partials than 256 x 256 tiles need to fill the GPU (MI355X, over 8192: 512 x 2048 30 against 43
+// us, 1000 x 2048 45 against 53; at 256 tiles, 2000 x 2048, 76 against 77).
 bool mid_small(int64_t m, int64_t n, int64_t ktot) {
     return m >= kMaterializeRows && ktot < 16384 && cdiv(m, 128) * cdiv(n, 128) <= 128;
 }
@@ -1387,9 +1392,7 @@ int mid_splits(int64_t m, int64_t n, int64_t ktot) {
     const int64_t tiles = cdiv(m, 256) * cdiv(n, 256);
     if (m >= kMaterializeRows && (ktot < kLongReduction || tiles >= 256)) return 1;
     if (mid_small(m, n, ktot)) {
-        const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
-        int64_t s = 256 / t128;
-        if (s < 4) s = 4;
+        int64_t s = balanced_splits(cdiv(m, 128) * cdiv(n, 128));
         const int64_t cap = cdiv(ktot, kBK) / 8;
         if (s > cap) s = cap;
         return (int)(s > 32 ? 32 : (s < 1 ? 1 : s));
@@ -1941,7 +1944,11 @@ namespace {
 // (17.5); 4001 x 64 over 4096 13.7 (24.1); 4001 x 256 over 8192 29.0 (47.4); dy b: 251 x 256
 // over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 with
 // 64 tiles or more, and under 4096 with 128 (a split costs more than it gains), outputs that fill
-// the grid of 128 x 128 tiles, and what split_repays_launch turns away.
+// the grid of 128 x 128 tiles, and what split_repays_launch turns away. The 256 x 256 split
+// route keeps what it runs faster: more than 128 columns in 48 tiles of 128 or more over 16384
+// and up (1030 x 1024 over 24576, both layouts, 67 and 78 us, 78 and 82 here; 4001 x 768 139 and
+// 167, 195 and 238), and in more than 128 tiles from kLongReduction on (3000 x 1024 over 8192 67
+// and 71, 67 and 86).
 // Wider outputs of up to 256 rows over the longest reductions (the loss's d hidden over its
 // vocabulary) split on 128 x 128 tiles to one workgroup per CU, where the route they took used
 // twice as many splits or 256-row tiles: 128 x 2048 over 49152 52 against 60 us, 128 x 4096 110
@@ -1967,10 +1974,14 @@ bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
         *splits = (int)least(256 / t128, mid_splits(m, n, k));  // the workspace is sized for the latter
         return *splits > 1;
     }
+    if (n > 128 && m >= kMaterializeRows && ((kt >= 256 && t128 >= 48) || (kt >= 128 && t128 > 128))) return false;
     int64_t s = 1;
-    if ((t64 > 128 && kt >= 64) || (t64 >= 128 && kt >= 128) || (t64 >= 32 && kt >= 256)) {
+    if ((t64 > 128 && kt >= 64) || (t64 >= (m < kMaterializeRows ? 128 : 64) && kt >= 128) ||
+        (t64 >= 32 && kt >= 256)) {
         *tile = TILE_128;
-        s = least(least((t128 >= 64 ? 512 : 256) / t128, kt / 16), t128 >= 64 ? 4 : (t128 >= 32 ? 8 : 24));
+        s = balanced_splits(t128);
+        if (s > kt / 16 && t128 > 64) s = 256 / t128;  // too short for two workgroups per CU
+        s = least(least(s, kt / 16), 24);
     } else {
         *tile = TILE_64;
         if (!((t64 >= 64 && kt < 32) || (t64 >= 128 && kt < 64))) {

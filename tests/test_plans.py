@@ -70,6 +70,16 @@ def test_rank_r_product_splits(m, n, k, splits):
     (4001, 64, 4096, 4),
     (4001, 256, 8192, 4),      # 128 x 128 tiles
     (16384, 256, 6144, 0),     # 256 tiles of 128 x 128 fill the GPU
+    # tiles of 128 x 128 in one workgroup per CU, or two past 64 of them
+    (520, 512, 12288, 12),     # 20 tiles
+    (1030, 1024, 12288, 7),    # 72
+    (3000, 512, 4096, 2),      # 96, too short for five parts
+    # more than 128 columns: the 256 x 256 route from 48 tiles over 16384, from 129 over 8192
+    (1500, 512, 16384, 21),    # 12 of 256 x 256
+    (1500, 384, 16384, 7),     # 36 of 128 x 128
+    (8192, 128, 16384, 4),     # no more than 128 columns
+    (3000, 1024, 8192, 5),     # 192 of 128 x 128: 48 of 256 x 256
+    (4096, 512, 8192, 4),      # 128
 ])
 def test_rank_r_product_splits_over_rows_and_reductions(m, n, k, splits):
     assert _gemm_ws(m, n, k) == splits * m * n * F32
@@ -77,6 +87,7 @@ def test_rank_r_product_splits_over_rows_and_reductions(m, n, k, splits):
 
 @pytest.mark.parametrize("m,n,k,splits", [
     (512, 2048, 8192, 4), (1000, 2048, 11008, 4), (513, 1032, 12288, 5),   # at most 128 tiles of 128 x 128
+    (520, 2048, 8192, 6),      # 80 of them: two workgroups per CU
     (2000, 2048, 8192, 4),     # 256 of them: the 256 x 256 route
 ])
 def test_long_reductions_into_small_outputs(m, n, k, splits):
