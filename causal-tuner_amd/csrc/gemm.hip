@@ -1971,7 +1971,7 @@ bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
     if (n > 1024) {
         if (m > 256 || kt < 256 || t128 > 32) return false;
         *tile = TILE_128;
-        *splits = (int)least(256 / t128, mid_splits(m, n, k));  // the workspace is sized for the latter
+        *splits = (int)least(256 / t128, mid_splits(m, n, k));  // no more than the route it replaces
         return *splits > 1;
     }
     if (n > 128 && m >= kMaterializeRows && ((kt >= 256 && t128 >= 48) || (kt >= 128 && t128 > 128))) return false;
@@ -2001,7 +2001,7 @@ extern "C" int64_t ct_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t tr
                                      int32_t c_dtype) {
     if (trans_a || c_dtype != CT_BF16) return 0;
     int tile, splits;
-    if (n <= 1024 && lowrank_split(m, n, k, &tile, &splits)) return lowrank_bytes(m, n, splits);
+    if (lowrank_split(m, n, k, &tile, &splits)) return lowrank_bytes(m, n, splits);
     const int64_t ks[2] = {k, 0};
     const int sb[2] = {trans_b ? SRC_KC : SRC_KS, trans_b ? SRC_KC : SRC_KS};
     return problem_workspace(m, n, ks, 1, sb);

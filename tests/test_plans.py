@@ -17,7 +17,11 @@ def _gemm_ws(m, n, k, trans_b=1):
 
 @pytest.mark.parametrize("m,n,k,splits", [
     # 65-511 rows: one round of 256 x 256 workgroups, at least 8 k-tiles per split, at most 32
-    (128, 2048, 49152, 32),    # the projection loss's d hidden per 128-row tile
+    (128, 2048, 49152, 16),    # the projection loss's d hidden per 128-row tile: 16 tiles of 128 x 128
+    (256, 2048, 16384, 8),     # the same in 32 of them, the most
+    (257, 2048, 49152, 16),    # a row more: 16 tiles of 256 x 256
+    (256, 2048, 16320, 31),    # a k-tile less (8 of 256 x 256)
+    (256, 2056, 16384, 28),    # 34 tiles of 128 (9 of 256)
     (256, 24576, 6144, 2),     # C5 at 256 rows, 96 output tiles
     (256, 6144, 24576, 10),    # C5 at 256 rows, 24 output tiles
     (384, 2048, 49152, 16),
