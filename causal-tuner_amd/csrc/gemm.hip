@@ -2153,10 +2153,10 @@ extern "C" int64_t ct_forward_linear_workspace(int64_t m, int64_t n, int64_t k, 
     return materialize_kind(nf4, m, n, k + r, kMaterializeRows) ? weight_bytes(n, k) + rest : rest;
 }
 
-// What the static-scratch entry point measures a problem by (ct_forward_linear_static): the
-// decoded weight and the larger of the base product's split partials and of the rank-r product's
-// in its simplest plans. More room only lets ct_gemm pick a faster plan, so a caller near the
-// limit keeps the calls it was given.
+// The size by which ct_forward_linear_static accepts a problem, as the header states it: the
+// decoded weight and the larger of the base product's split partials and of the rank-r product's,
+// the latter by a fixed formula. It is a limit, not a plan: what runs is ct_gemm's own choice in
+// the room there is, so a faster plan that asks for more turns no call away.
 namespace ct {
 int64_t forward_linear_scratch(int64_t m, int64_t n, int64_t k, int64_t r, int32_t nf4) {
     int64_t inner;

@@ -1,7 +1,7 @@
 // ct_forward_linear_static: ct_forward_linear for callers that cannot allocate device
-// memory (tight serving loops, harnesses that forbid hipMalloc). Its scratch space -- the split partials of few-row problems and, from 512 rows
-// on, the decoded bf16 weight -- lives in one file-scope device array of
-// CT_STATIC_SCRATCH_BYTES per GPU instead of a caller's workspace. The array is created
+// memory (tight serving loops, harnesses that forbid hipMalloc). Its scratch space -- the split
+// partials and, from 512 rows on, the decoded bf16 weight -- lives in one file-scope device
+// array of CT_STATIC_SCRATCH_BYTES per GPU instead of a caller's workspace. The array is created
 // when the library's code object loads on a device and held until the process ends.
 //
 // Host code never passes the array's name to a kernel: on the host that name is only a
@@ -68,7 +68,7 @@ extern "C" int ct_forward_linear_static(const void *x, int64_t ldx, const void *
     const int32_t kind = w_nf4 ? (w_nf4->nested ? 1 : 2) : 0;
     const int64_t need = ct::forward_linear_scratch(m, n, k, r, kind);
     if (need < 0 || need > (int64_t)CT_STATIC_SCRATCH_BYTES) return -CT_EINVAL_WORKSPACE;
-    // The preferred plans may use more (up to the whole array); what does not fit runs unsplit.
+    // The preferred plans may use more (up to the whole array); what does not fit splits less.
     const int64_t want = ct_forward_linear_workspace(m, n, k, r, kind);
     const int64_t room = want < (int64_t)CT_STATIC_SCRATCH_BYTES ? want : (int64_t)CT_STATIC_SCRATCH_BYTES;
     void *ws = nullptr;

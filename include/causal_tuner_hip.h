@@ -183,14 +183,15 @@ int ct_nf4_quantize(const void *w, int32_t w_dtype, int64_t n, int32_t blocksize
  *   B(k,n) = b[n*ldb + k]  (trans_b = 1)  or  b[k*ldb + n]  (trans_b = 0)
  * c_dtype is CT_BF16 (rounded once, RTNE) or CT_F32. bias may be null (bf16 [n]).
  *
- * Workspace (here and in ct_forward_linear / ct_input_gradient): with m <= 64 rows, with
- * 65-511 rows, with a rank-r output (n <= 1024) over many rows and a reduction of at least
- * 4096, and with a reduction of at least 8192 into an output short of one round of
- * 256 x 256 tiles, the reduction may be split across workgroups, the fp32 partials going to the caller's
- * workspace and summed in a fixed order (results do not depend on timing). The *_workspace
- * query gives the size that allows the preferred split; a null or smaller workspace is
- * valid and only splits less (no split at all without one). The partials are written with
- * 16-byte stores, so a workspace that is not 16-byte aligned is treated as absent.
+ * Workspace (here and in ct_forward_linear / ct_input_gradient): with up to 511 rows, with a
+ * rank-r output (n <= 1024) over more of them where the split repays its second launch, and
+ * with a reduction of at least 8192 into an output short of one round of 256 x 256 tiles, the
+ * reduction may be split across workgroups, the fp32 partials going to the caller's workspace
+ * and summed in a fixed order (results do not depend on timing), bias and beta added once after
+ * the sum. The *_workspace query gives the size that allows the preferred split; a null or
+ * smaller workspace is valid and only splits less (no split at all without one), which changes
+ * the order of the sums. The partials are written with 16-byte stores, so a workspace that is
+ * not 16-byte aligned is treated as absent.
  */
 int64_t ct_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t trans_a, int32_t trans_b, int32_t c_dtype);
 int ct_gemm(const void *a, int64_t lda, int32_t trans_a,
@@ -201,8 +202,12 @@ int ct_gemm(const void *a, int64_t lda, int32_t trans_a,
 /*
  * The same products for a float32 compute dtype (the reference's torch.mm / addmm with
  * float32 operands, kernels/linear.py:16-44, TF32 off as in train.py:80-82): float32 a, b,
- * c and bias, fp32 MFMA products and sums (v_mfma_f32_16x16x4_f32), one in-order reduction
- * over k per output element (deterministic). Layouts as ct_gemm:
+ * c and bias, fp32 MFMA products and sums (v_mfma_f32_16x16x4_f32), reduced over k in a fixed
+ * order (deterministic). The order depends on the sizes: one chain in index order, except that
+ * an output of fewer than 256 tiles of 64 x 64 over more than 128 indices is summed in eight
+ * interleaved parts, added in order, so rows computed in calls of other sizes may differ in
+ * the last bits. Each operand takes 16-byte loads where its base is 16-byte aligned and its
+ * pitch a multiple of 4. Layouts as ct_gemm:
  *   c[m,n] = sum_k A(m,k) B(k,n) (+ bias[n]) (+ c[m,n] if beta)
  * With beta = 0, c is only written. No workspace.
  */
@@ -329,15 +334,19 @@ int ct_forward_linear(const void *x, int64_t ldx,
  * ct_forward_linear without a workspace argument, for callers that cannot allocate device
  * memory (tight serving loops, harnesses that forbid hipMalloc). No counterpart in the
  * reference, whose operators allocate their workspaces with torch (kernels/linear.py:67,74).
- * Same arguments, results and row regimes as ct_forward_linear, which it calls with the
- * library's static device scratch array of CT_STATIC_SCRATCH_BYTES per GPU (held from the
- * library's load on that GPU until the process ends) in place of the workspace. Its device
- * address is resolved once per GPU by ct_init_device (or, on a GPU never set up, by the
- * first static call there). A problem whose ct_forward_linear_workspace exceeds
- * CT_STATIC_SCRATCH_BYTES returns -CT_EINVAL_WORKSPACE before anything is enqueued: 64 MiB
- * covers every few-row problem and the many-row ones whose decoded weight, plus the
- * split partials where the reduction is split, fits (up to about 32 M weight elements
- * without a split). It calls no allocator. Every call on one GPU uses that GPU's
+ * Same arguments and row regimes as ct_forward_linear, which it calls with the library's
+ * static device scratch array of CT_STATIC_SCRATCH_BYTES per GPU (held from the library's load
+ * on that GPU until the process ends) as the workspace: min(ct_forward_linear_workspace,
+ * CT_STATIC_SCRATCH_BYTES) bytes of it, with the results of ct_forward_linear given as many.
+ * (Where the query exceeds the array, xa = x a^T finds less room than its preferred split
+ * needs and is summed in another order.) The array's device address is resolved once per GPU
+ * by ct_init_device (or, on a GPU never set up, by the first static call there). A problem
+ * returns -CT_EINVAL_WORKSPACE before anything is enqueued when its decoded weight, plus the
+ * larger of the base product's split partials and xa's, exceeds CT_STATIC_SCRATCH_BYTES; xa's
+ * count as 2 to 4 splits from 4096 rows over 4096 and up, elsewhere as the splits of a 256 x
+ * 256-tile product. 64 MiB covers every few-row problem and the many-row ones whose decoded
+ * weight fits beside the partials (up to about 32 M weight elements without a split). It calls
+ * no allocator. Every call on one GPU uses that GPU's
  * one array: calls that overlap on a GPU (two streams or threads) race and must be ordered
  * by the caller. Capture of these calls into a HIP graph is not supported.
  */
