@@ -5,7 +5,8 @@ kernels/linear.py:90-91, kernels/mlp_cuda.py:80), SiLU x up and its backward
 (kernels/core_cuda.py:133-200).
 
 Every route of the GEMM is covered -- the few-row kernels (<= 64 rows), the split 256 x 256
-runner (65..511 rows with a small output), the 64/128/256 tiles, a row pitch that is not a
+runner (65..511 rows with a small output), the 64/128/256 tiles, the 256 x 256 tile kept at
+65..511 rows (an NF4 base is decoded between its products there), a row pitch that is not a
 multiple of 8, dense and NF4 bases -- and each must give the unfused sequence's values bit
 for bit: both apply the same device functions to the same bf16-rounded projection output.
 The operator-level tests run the q/k/v group and the MLP with the fusion on and off
@@ -17,9 +18,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 # (rows, out features, in features): few-row kernels, split runner, 64 tiles, 128 tiles,
-# 256 tiles, unaligned output pitch
+# 256 tiles, unaligned output pitch, 256 tiles at few rows
 ROUTES = [(16, 1024, 2048), (48, 512, 1024), (130, 1024, 2048), (300, 4096, 512), (2048, 2048, 1024),
-          (4096, 4096, 512), (77, 1004, 256)]
+          (4096, 4096, 512), (77, 1004, 256), (400, 20096, 512)]
 
 
 def _base(k, n, r, nf4, seed):

@@ -75,12 +75,17 @@ def test_fused_forward_and_input_gradient_equal_materialized(m, k, n, r):
 
 
 @pytest.mark.parametrize("m,k,n,r", [
-    (66, 64, 72, 8), (128, 128, 256, 8), (251, 192, 520, 24), (255, 4160, 264, 40), (300, 320, 1000, 8),
-    (65, 24576, 520, 256), (257, 8256, 2048, 16), (511, 8192, 776, 72)])
+    # unsplit on 64 x 64 tiles, whose step decodes a k-tile at once
+    (66, 64, 72, 8), (128, 128, 256, 8), (251, 192, 520, 24), (300, 320, 1000, 8),
+    # the 256 x 256 step that spreads the decode over its columns: 8 to 16 k-tiles of a split,
+    (255, 4160, 264, 40), (65, 24576, 520, 256), (257, 8256, 2048, 16), (511, 8192, 776, 72),
+    # and unsplit (too few tiles of 256 for the CUs, too many of 128 for one round) over 1, 2, 5 and 8
+    (511, 64, 16640, 8), (257, 96, 22016, 8), (300, 320, 24584, 24), (400, 512, 20000, 256)])
 @pytest.mark.parametrize("nested", [False, True])
 def test_decode_between_the_products_changes_no_bit(m, k, n, r, nested):
-    """65 - 511 rows: the 256 x 256 k-step that spreads the decode over its columns, from one
-    k-tile to 384, odd and even counts, with and without splits, against the dense weight."""
+    """65 - 511 rows over a packed weight, with a bias, on every route of the forward, against the
+    dense weight, bit for bit (a weight without double quantization takes the element-wise
+    decode where it is not split, and is decoded first where it is)."""
     packed, state = _weight(n, k, nested=nested, seed=m)
     dense = materialize(packed, state, torch.bfloat16)
     x, a, b, _, bias = _inputs(m, k, n, r, seed=n)
