@@ -235,3 +235,27 @@ def test_contiguous_quantizer_codes_every_value_as_the_oracle(count, blocksize, 
         at = 3 * blocksize + 2
         byte = int(packed.cpu().view(-1)[at // 2])
         assert (byte >> 4 if at % 2 == 0 else byte & 15) == 15
+
+
+@pytest.mark.parametrize("first,last", [(-0.2, 0.2), (-0.9, 0.99), (-1.5, 1.5)])
+def test_quantizer_takes_midpoints_its_cell_table_cannot_hold(first, last):
+    """The contiguous kernel's table holds at most one midpoint per 1/16 of [-1, 1] and none in
+    the last; other midpoints (here several to a cell, one in the last, some outside) are
+    compared one by one: code = the number of midpoints below x, in fp32."""
+    from causal_tuner.kernels import _native
+    lib = _native.library()
+    g = torch.Generator().manual_seed(7)
+    mids = torch.linspace(first, last, 15)
+    values = torch.rand(64 * 130, generator=g) * 2 - 1
+    values[::64] = 1.0
+    values[1:16], values[65:80] = mids.clamp(-1, 1), torch.nextafter(mids, mids - 1).clamp(-1, 1)
+    device = [t.cuda() for t in (values, mids)]
+    packed = torch.empty(len(values) // 2, dtype=torch.uint8, device="cuda")
+    absmax = torch.empty(130, device="cuda")
+    status = lib.ct_nf4_quantize(device[0].data_ptr(), _native.CT_F32, len(values), 64, 0, device[1].data_ptr(), None,
+                                 packed.data_ptr(), absmax.data_ptr(), None, None, None, 0, _native.stream_of(packed))
+    assert status == 0
+    scaled = (values.view(130, 64) * (1.0 / values.view(130, 64).abs().amax(1, keepdim=True))).view(-1, 1)
+    codes = (~(mids[None] >= scaled)).sum(1).to(torch.uint8).view(-1, 2)
+    assert torch.equal(packed.cpu(), codes[:, 0] << 4 | codes[:, 1])
+    assert torch.equal(absmax.cpu(), values.view(130, 64).abs().amax(1))
