@@ -704,8 +704,10 @@ struct FastRunner {
     // over the columns, each piece's code-book reads two columns ahead of its products, and
     // every column's order is fixed, so that lookups, conversions and stores run between the
     // MFMAs. Left to the scheduler (step above, whose group pattern does not know the lookups)
-    // the phases ran one after the other: MFMA 29%, VALU 28% and LDS 40% busy, none of them
-    // bound (251 rows, 24576 -> 6144: 116 us, 106 here; 128 rows 94, 82). Same values and sums.
+    // the phases ran one after the other, no unit near its bound (MFMA 29% busy). MI355X, the
+    // launch with its split reduction, with the step above and here: 251 rows, 24576 -> 6144 112
+    // and 102 us, 6144 -> 24576 130 and 113, 128 rows 101 and 88, 4096 -> 4096 37 and 34. Same
+    // values and sums.
     template <int J>
     __device__ __forceinline__ static void packed_column(LA &la, const LB &now, const uint4 *cur, uint4 *nxt,
                                                          const uint4 (&af)[KS][FM], uint4 (&bf)[2][KS],
@@ -1430,11 +1432,12 @@ int operand_segments(const GemmParams &p) { return p.group_tiles > 0 ? 2 : p.nse
 // Columns of segment s's B operand.
 int64_t segment_cols(const GemmParams &p, int s) { return (p.group_tiles > 0 && s == 1) ? p.n1 : p.n; }
 
-// Vector (16-byte) operand access needs aligned bases, leading dimensions that are
-// multiples of 8 elements, and 8-multiple extents along each contiguous dimension.
 // Sources that read 8 (KC) or 32 (NF4) consecutive reduction indices at once.
 constexpr bool along_reduction(int src) { return src == SRC_KC || src == SRC_NF4; }
 
+// Vector (16-byte) operand access needs aligned bases, leading dimensions that are
+// multiples of 8 elements, and a multiple of 8 elements along the dimension that an operand's
+// chunks run along: the reduction or the output's rows or columns.
 bool vec_ok(const Problem &pr) {
     const GemmParams &p = pr.p;
     for (int s = 0; s < operand_segments(p); ++s) {
@@ -1940,9 +1943,9 @@ namespace {
 // tiles take over where the rows and the reduction are long. Fitted to a sweep on MI355X of
 // 100 - 8192 rows, 16 - 512 columns and reductions of 1024 - 24576, both layouts, over tiles of
 // 64, 128 and 256 with 1 - 32 splits; x a^T, us now (and on the 256 x 256 split or unsplit 64 x
-// 64 grid before): 251 x 256 over 2048 8.2 (19.3), over 24576 19 (28); 1000 x 256 over 4096 12.0
-// (17.5); 4001 x 64 over 4096 13.7 (24.1); 4001 x 256 over 8192 29.0 (47.4); dy b: 251 x 256
-// over 2048 9.3 (23.1), 4001 x 256 over 8192 35.0 (45.9). Left alone: reductions under 2048 with
+// 64 grid before): 251 x 256 over 2048 7.9 (18.7), over 24576 17.3 (28.5); 4001 x 64 over 4096
+// 14.3 (24.4); 4001 x 256 over 8192 30.6 (43.0); dy b: 251 x 256 over 2048 8.8 (22.3), 4001 x
+// 256 over 8192 32.4 (44.8). Left alone: reductions under 2048 with
 // 64 tiles or more, and under 4096 with 128 (a split costs more than it gains), outputs that fill
 // the grid of 128 x 128 tiles, and what split_repays_launch turns away. The 256 x 256 split
 // route keeps what it runs faster: more than 128 columns in 48 tiles of 128 or more over 16384
@@ -1951,8 +1954,8 @@ namespace {
 // and 71, 67 and 86).
 // Wider outputs of up to 256 rows over the longest reductions (the loss's d hidden over its
 // vocabulary) split on 128 x 128 tiles to one workgroup per CU, where the route they took used
-// twice as many splits or 256-row tiles: 128 x 2048 over 49152 52 against 60 us, 128 x 4096 110
-// against 120, 256 x 2048 80 against 87.
+// twice as many splits or 256-row tiles: 128 x 2048 over 49152 46 against 61 us, 128 x 4096 107
+// against 121, 256 x 2048 76 against 89 (with the order by split and the second register set).
 // A split adds a launch, which costs a step that the host bounds about 4 us per product whatever it
 // saves on the GPU. Below kMaterializeRows the route it replaces splits as well, and so it does
 // from kLongReduction on. Between, a projection (m rows, k x k) occupies the GPU for less time
