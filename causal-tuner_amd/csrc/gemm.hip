@@ -1945,7 +1945,9 @@ namespace {
 // 64, 128 and 256 with 1 - 32 splits; x a^T, us now (and on the 256 x 256 split or unsplit 64 x
 // 64 grid before): 251 x 256 over 2048 7.9 (18.7), over 24576 17.3 (28.5); 4001 x 64 over 4096
 // 14.3 (24.4); 4001 x 256 over 8192 30.6 (43.0); dy b: 251 x 256 over 2048 8.8 (22.3), 4001 x
-// 256 over 8192 32.4 (44.8). Left alone: reductions under 2048 with
+// 256 over 8192 32.4 (44.8). dy b stops at 256 workgroups of 64 x 64: 49 sizes of 65 - 511 rows
+// 0.84 of the time in 512, which was up to 1.33 of the 256 x 256 split's (256 x 256 over 24576 in
+// 16 splits 16.9, in 24 21.2 us); x a^T gains from the larger count (1.09 in 256). Left alone: reductions under 2048 with
 // 64 tiles or more, and under 4096 with 128 (a split costs more than it gains), outputs that fill
 // the grid of 128 x 128 tiles, and what split_repays_launch turns away. The 256 x 256 split
 // route keeps what it runs faster: more than 128 columns in 48 tiles of 128 or more over 16384
@@ -1967,7 +1969,7 @@ bool split_repays_launch(int64_t m, int64_t k) {
     if (m < kMaterializeRows || k >= kLongReduction) return true;
     return k >= 4096 && (double)m * (double)k * (double)k >= 4e10;
 }
-bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
+bool lowrank_split(int64_t m, int64_t n, int64_t k, bool trans_b, int *tile, int *splits) {
     const int64_t t64 = cdiv(m, 64) * cdiv(n, 64), t128 = cdiv(m, 128) * cdiv(n, 128), kt = cdiv(k, kBK);
     const auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
     if (m <= 64 || n <= 0 || t128 >= 256 || !split_repays_launch(m, k)) return false;
@@ -1989,7 +1991,8 @@ bool lowrank_split(int64_t m, int64_t n, int64_t k, int *tile, int *splits) {
         *tile = TILE_64;
         if (!((t64 >= 64 && kt < 32) || (t64 >= 128 && kt < 64))) {
             const int64_t deep = least(512 / t64, kt / 16), wide = least(256 / t64, kt / 8);
-            s = least(deep > wide ? deep : wide, 24);
+            // dy b has its second register set up to 256 workgroups only (launch_cfg)
+            s = least(deep > wide && (trans_b || t64 >= 64) ? deep : wide, 24);
         }
     }
     *splits = (int)(s < 1 ? 1 : s);
@@ -2004,7 +2007,7 @@ extern "C" int64_t ct_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t tr
                                      int32_t c_dtype) {
     if (trans_a || c_dtype != CT_BF16) return 0;
     int tile, splits;
-    if (lowrank_split(m, n, k, &tile, &splits)) return lowrank_bytes(m, n, splits);
+    if (lowrank_split(m, n, k, trans_b != 0, &tile, &splits)) return lowrank_bytes(m, n, splits);
     const int64_t ks[2] = {k, 0};
     const int sb[2] = {trans_b ? SRC_KC : SRC_KS, trans_b ? SRC_KC : SRC_KS};
     return problem_workspace(m, n, ks, 1, sb);
@@ -2038,7 +2041,7 @@ extern "C" int ct_gemm(const void *a, int64_t lda, int32_t trans_a, const void *
     pr.ws_bytes = workspace ? workspace_bytes : 0;
     pr.vec = vec_ok(pr);
     int tile, splits;
-    if (c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, &tile, &splits) &&
+    if (c_dtype == CT_BF16 && !trans_a && lowrank_split(m, n, k, trans_b != 0, &tile, &splits) &&
         (splits == 1 || (workspace && aligned16(workspace))) && pr.ws_bytes >= lowrank_bytes(m, n, splits)) {
         pr.tile = tile;
         pr.splits = splits;

@@ -89,6 +89,15 @@ def test_rank_r_product_splits_over_rows_and_reductions(m, n, k, splits):
     assert _gemm_ws(m, n, k) == splits * m * n * F32
 
 
+@pytest.mark.parametrize("m,n,k,trans_b,splits", [
+    (128, 512, 24576, 1, 24), (128, 512, 24576, 0, 16),   # 16 tiles of 64 x 64
+    (511, 448, 12288, 1, 9), (511, 448, 12288, 0, 4),     # 56
+    (511, 512, 12288, 1, 8), (511, 512, 12288, 0, 8),     # 64: 512 workgroups either way
+])
+def test_rank_r_products_past_one_workgroup_per_cu(m, n, k, trans_b, splits):
+    assert _gemm_ws(m, n, k, trans_b) == splits * m * n * F32
+
+
 @pytest.mark.parametrize("m,n,k,splits", [
     (512, 2048, 8192, 4), (1000, 2048, 11008, 4), (513, 1032, 12288, 5),   # at most 128 tiles of 128 x 128
     (520, 2048, 8192, 6),      # 80 of them: two workgroups per CU
