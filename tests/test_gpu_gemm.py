@@ -265,6 +265,8 @@ def test_partial_last_round_column_split_in_the_input_gradient():
 @pytest.mark.parametrize("m,n,k", [
     (65, 8, 64), (65, 16, 8192), (251, 256, 2048), (251, 250, 2040), (511, 512, 1024), (513, 72, 4096), (1000, 256, 4096),
     (4001, 64, 4096), (4001, 256, 8192), (500, 512, 16448),      # rank-r products: every tile and split rule
+    (1030, 1016, 12288), (3000, 512, 4096), (1500, 520, 16384), (3000, 1000, 8200),   # two workgroups per CU, or 256 x 256
+    (520, 2048, 8192),                                           # 80 tiles of 128 x 128
     (128, 1216, 16384), (77, 4096, 16448), (256, 2048, 20000),   # up to 256 rows over the longest reductions
     (513, 1032, 12288), (1000, 2048, 8200)])                     # from 512 rows on 128 x 128 tiles
 def test_planned_products_against_float64(m, n, k, trans_b):
